@@ -377,31 +377,54 @@ g4::TokArgs tok_args(const g4_weight *w, int64_t off, const float *d_X, int32_t 
   return t;
 }
 
-// Scratch floats batch_dev needs for partial sums (carved by the caller).
-int64_t batch_part_floats(const g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0,
-                          int32_t dim1) {
-  if (M < 3 || dim0 == 0 || dim1 == 0) return 0;
+// How a batched call runs, and the scratch floats it needs for partial sums.
+struct BatchRoute {
+  enum Kind { ROWS, TOK, MAT } kind;
+  int64_t part;
+};
+
+// Several tokens of one matrix: the matrix-core kernels unpack each weight once
+// for 16 of them (Q4_K: g4_tok.hip, the other formats: g4_mat.hip); the row engine
+// runs one segment per token.
+BatchRoute batch_route(const g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1) {
+  if (M < 3 || dim0 == 0 || dim1 == 0) return {BatchRoute::ROWS, 0};
   const g4::TokArgs t = tok_args(w, off, nullptr, M, nullptr, dim0, dim1);
-  return g4::tok_ok(w->type, t) ? g4::tok_scratch_floats(t, ctx->dev) : 0;
+  // Two tokens stay on the row engine: measured on 8192 x 2048 Q4_K, 6.5 us against
+  // 8.9 us for the matrix cores; from three on the matrix cores are as fast or
+  // faster (9.1 / 9.3 us at M = 3, 9.6 / 14.4 at M = 8).  For the other formats
+  // mat_min_tokens draws the line.
+  if (g4::tok_ok(w->type, t)) return {BatchRoute::TOK, g4::tok_scratch_floats(t, ctx->dev)};
+  if (M >= g4::mat_min_tokens(w->type, t) && g4::mat_ok(w->type, t))
+    return {BatchRoute::MAT, g4::mat_scratch_floats(t, ctx->dev)};
+  return {BatchRoute::ROWS, 0};
+}
+
+// The route of a call that needs `before` bytes of scratch besides, with that
+// scratch there.  A call of the formats the row engine takes without scratch
+// falls back to it where no scratch can be had (none reserved under a capture, no
+// memory left).
+int batch_prepare(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1, size_t before,
+                  BatchRoute *r) {
+  *r = batch_route(ctx, w, off, M, dim0, dim1);
+  const int rc = ensure_scratch(ctx, before + sizeof(float) * (size_t)r->part);
+  if (rc == G4_OK || r->kind != BatchRoute::MAT || r->part == 0) return rc;
+  *r = {BatchRoute::ROWS, 0};
+  return ensure_scratch(ctx, before);
 }
 
 int batch_dev(g4_ctx *ctx, const g4_weight *w, int64_t off, const float *d_X, int32_t M, float *d_Y, int32_t dim0,
-              int32_t dim1, float *d_part) {
+              int32_t dim1, const BatchRoute &r, float *d_part) {
   if (dim0 == 0 || M == 0) return G4_OK;
   if (dim1 == 0) {
     G4_TRY(zero_dev(ctx, d_Y, sizeof(float) * (size_t)dim0 * M));
     return G4_OK;
   }
-  // several tokens: the matrix-core kernel unpacks each weight once for all of
-  // them.  Two tokens stay on the row engine (one segment each): measured on
-  // 8192 x 2048, 6.5 us against 8.9 us for the matrix cores; from three on the
-  // matrix cores are as fast or faster (9.1 / 9.3 us at M = 3, 9.6 / 14.4 at M = 8).
-  if (M >= 3) {
+  if (r.kind != BatchRoute::ROWS) {
     g4::TokArgs t = tok_args(w, off, d_X, M, d_Y, dim0, dim1);
-    if (g4::tok_ok(w->type, t)) {
-      t.part = d_part;
-      return launch_status(g4::launch_tok(w->type, t, ctx->dev, ctx->stream), "matmul_batch");
-    }
+    t.part = r.part > 0 ? d_part : nullptr;
+    return launch_status(r.kind == BatchRoute::TOK ? g4::launch_tok(w->type, t, ctx->dev, ctx->stream)
+                                                   : g4::launch_mat(w->type, t, ctx->dev, ctx->stream),
+                         "matmul_batch");
   }
   g4::RowsArgs a = plain_rows(w, off, d_X, d_Y, dim0, dim1);
   a.x_stride = dim1;
@@ -979,11 +1002,12 @@ int g4_matmul_batch(g4_ctx *ctx, const g4_weight *w, int64_t this_offset, const 
   G4_TRY(use_host(ctx));
   Carve c;
   size_t ox = c.add(sizeof(float) * (size_t)dim1 * M), oy = c.add(sizeof(float) * (size_t)dim0 * M);
-  size_t op = c.add(sizeof(float) * (size_t)batch_part_floats(ctx, w, this_offset, M, dim0, dim1));
-  G4_TRY(ensure_scratch(ctx, c.off));
+  const size_t op = c.add(0);
+  BatchRoute r;
+  G4_TRY(batch_prepare(ctx, w, this_offset, M, dim0, dim1, op, &r));
   float *dx = (float *)(ctx->scratch + ox), *dy = (float *)(ctx->scratch + oy), *dp = (float *)(ctx->scratch + op);
   G4_TRY(copy_in(ctx, dx, X, sizeof(float) * (size_t)dim1 * M));
-  G4_TRY(batch_dev(ctx, w, this_offset, dx, M, dy, dim0, dim1, dp));
+  G4_TRY(batch_dev(ctx, w, this_offset, dx, M, dy, dim0, dim1, r, dp));
   G4_TRY(copy_out(ctx, Y, dy, sizeof(float) * (size_t)dim0 * M));
   return finish(ctx);
 }
@@ -998,9 +1022,9 @@ int g4_matmul_batch_dev(g4_ctx *ctx, const g4_weight *w, int64_t this_offset, co
   if ((!d_X && M > 0 && dim1 > 0) || (!d_Y && M > 0 && dim0 > 0))
     return fail(G4_ERR_INVALID_ARGUMENT, "X/Y is null");
   G4_TRY(use_device(ctx));
-  const int64_t pf = batch_part_floats(ctx, w, this_offset, M, dim0, dim1);
-  if (pf > 0) G4_TRY(ensure_scratch(ctx, sizeof(float) * (size_t)pf));
-  return batch_dev(ctx, w, this_offset, d_X, M, d_Y, dim0, dim1, pf > 0 ? (float *)ctx->scratch : nullptr);
+  BatchRoute r;
+  G4_TRY(batch_prepare(ctx, w, this_offset, M, dim0, dim1, 0, &r));
+  return batch_dev(ctx, w, this_offset, d_X, M, d_Y, dim0, dim1, r, (float *)ctx->scratch);
 }
 
 // -------------------------------------------------------------- argmax ----

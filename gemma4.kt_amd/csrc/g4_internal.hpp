@@ -97,6 +97,15 @@ bool tok_ok(int type, const TokArgs &a);
 // Scratch the launch needs for partial sums (0: one column split, y written directly).
 int64_t tok_scratch_floats(const TokArgs &a, const DevInfo &dev);
 hipError_t launch_tok(int type, const TokArgs &a, const DevInfo &dev, hipStream_t stream);
+// y[m * y_stride + r] = the sum over `splits` partial results part[split][m][r], in split order
+hipError_t launch_tok_reduce(const float *part, int splits, int32_t M, int32_t rows, float *y, int64_t y_stride,
+                             hipStream_t stream);
+// The same matmul for the other block formats and for BF16 and F16 (g4_mat.hip).
+bool mat_ok(int type, const TokArgs &a);
+// The fewest tokens it is the faster route for.
+int32_t mat_min_tokens(int type, const TokArgs &a);
+int64_t mat_scratch_floats(const TokArgs &a, const DevInfo &dev);
+hipError_t launch_mat(int type, const TokArgs &a, const DevInfo &dev, hipStream_t stream);
 
 // Routed experts of a multi-token MoE call on the matrix cores, grouped by
 // expert (Q4_K): pair p = (token p / x_div, slot p % x_div) with expert ids[p]

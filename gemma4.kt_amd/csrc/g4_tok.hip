@@ -43,7 +43,7 @@
 // adds in split order.  Splitting the columns this way keeps the x each
 // workgroup loads and splits to its own share, so the split work does not grow
 // with the number of workgroups.
-#include "g4_device.hpp"
+#include "g4_mmfmt.hpp"
 #include "g4_internal.hpp"
 
 #include <algorithm>
@@ -51,41 +51,9 @@
 
 namespace g4 {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
 
 constexpr int TOK_SLOTS = 4;  // (token tile, 64-column group) pairs a wave can keep split in registers
-
-// x = p1 + p2 + p3 exactly: p1 and p2 are the bf16 truncations of x and of
-// x - p1 (their top 8 significant bits), x - p1 - p2 has at most 8 significant
-// bits, and both differences are exact in fp32.  Truncation keeps every part of
-// a finite x finite.  GUARD: an infinite x stays in p1 with zero residuals;
-// without it x - p1 is NaN there, which the caller detects.  A NaN x gives NaN
-// parts either way.
-template <bool GUARD>
-G4_DEV void split3(const float (&v)[8], bf16x8 &p1, bf16x8 &p2, bf16x8 &p3) {
-  uint32_t t1[8], t2[8], t3[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    t1[e] = __float_as_uint(v[e]) & 0xFFFF0000u;
-    float r1 = v[e] - __uint_as_float(t1[e]);
-    if (GUARD) r1 = __builtin_isinf(v[e]) ? 0.f : r1;
-    t2[e] = __float_as_uint(r1) & 0xFFFF0000u;
-    t3[e] = __float_as_uint(r1 - __uint_as_float(t2[e]));
-  }
-  // two values' upper halves per dword (v_perm_b32)
-  u32x4 a, b, c;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    a[k] = __builtin_amdgcn_perm(t1[2 * k + 1], t1[2 * k], 0x07060302u);
-    b[k] = __builtin_amdgcn_perm(t2[2 * k + 1], t2[2 * k], 0x07060302u);
-    c[k] = __builtin_amdgcn_perm(t3[2 * k + 1], t3[2 * k], 0x07060302u);
-  }
-  p1 = __builtin_bit_cast(bf16x8, a);
-  p2 = __builtin_bit_cast(bf16x8, b);
-  p3 = __builtin_bit_cast(bf16x8, c);
-}
 
 // split3 for four values: parts p = 0, 1, 2 as two dwords each (values 0, 1
 // and 2, 3 in the low and high halves), the same parts as split3 gives
@@ -711,17 +679,21 @@ hipError_t launch_tok(int type, const TokArgs &a, const DevInfo &dev, hipStream_
     hipLaunchKernelGGL((k_tok_q4k<TOK_TT, TOK_WPB, false, false, true, false>), grid, dim3(TOK_WPB * 64), 0, s, a);
   else
     hipLaunchKernelGGL((k_tok_q4k<TOK_TT, TOK_WPB, false, false, false, false>), grid, dim3(TOK_WPB * 64), 0, s, a);
-  if (sh.splits == 1) return hipGetLastError();
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || sh.splits == 1) return e;
+  return launch_tok_reduce(a.part, sh.splits, a.M, a.rows, a.y, a.y_stride, s);
+}
+
+hipError_t launch_tok_reduce(const float *part, int splits, int32_t M, int32_t rows, float *y, int64_t y_stride,
+                             hipStream_t s) {
   // four rows per thread when every row quad and its output are 16-byte aligned
   // (the scratch is; y depends on the caller)
-  if ((a.rows % 4) == 0 && (a.y_stride % 4) == 0 && ((uintptr_t)a.y & 15) == 0)
-    hipLaunchKernelGGL(k_tok_reduce<4>, dim3((unsigned)((a.rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, s,
-                       (const float *)a.part, sh.splits, a.M, a.rows, a.y, a.y_stride);
+  if ((rows % 4) == 0 && (y_stride % 4) == 0 && ((uintptr_t)y & 15) == 0)
+    hipLaunchKernelGGL(k_tok_reduce<4>, dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)M), dim3(256), 0, s, part,
+                       splits, M, rows, y, y_stride);
   else
-    hipLaunchKernelGGL(k_tok_reduce<1>, dim3((unsigned)((a.rows + 255) / 256), (unsigned)a.M), dim3(256), 0, s,
-                       (const float *)a.part, sh.splits, a.M, a.rows, a.y, a.y_stride);
+    hipLaunchKernelGGL(k_tok_reduce<1>, dim3((unsigned)((rows + 255) / 256), (unsigned)M), dim3(256), 0, s, part,
+                       splits, M, rows, y, y_stride);
   return hipGetLastError();
 }
 

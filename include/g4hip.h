@@ -86,7 +86,8 @@ int g4_ctx_device(const g4_ctx *ctx, int *ordinal);
  *  - g4_ctx_reserve grows the buffer to `bytes` now (call it, or run the largest
  *    shapes once eagerly, before capturing);
  *  - a call that needs more than is reserved while its stream is capturing
- *    returns G4_ERR_INVALID_ARGUMENT and records nothing;
+ *    returns G4_ERR_INVALID_ARGUMENT and records nothing (g4_matmul_batch_dev of
+ *    the types other than Q4_K then records its slower kernels, which need none);
  *  - once any call on the context has been captured, an outgrown buffer is kept
  *    allocated (graphs may still replay into it) until g4_close.
  * Host-pointer calls synchronise and return G4_ERR_INVALID_ARGUMENT under capture.

@@ -257,3 +257,45 @@ def test_host_pointer_calls_are_refused_under_capture(g4, moe_weights):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+@pytest.mark.parametrize("reserve", [0, 8 << 20])
+def test_batched_wide_rows_captured(g4, reserve):
+    """Several tokens against rows of more than 2048 columns: the column splits' sums
+    need scratch.  Where none is reserved a captured call runs without it (one
+    segment of the row engine per token) instead of failing; with it the replays
+    give the eager bits."""
+    announce("capture: batched wide rows, %d bytes reserved" % reserve)
+    m, rows, cols = 12, 40, 4096
+    raw = synth.weights(46, "bw", 8, rows * cols)
+    X = torch.from_numpy(synth.activations(46, "bwx", m * cols).reshape(m, cols)).cuda()
+    Y = torch.empty((m, rows), device="cuda")
+    c = g4.Context(0)
+    stream = torch.cuda.Stream()
+    try:
+        w = g4.FloatTensorFactory.create(c, 8, raw, rows * cols)
+        w.matmul_batch_dev(X, 1, Y, rows, cols)  # (no scratch)
+        if reserve:
+            c.reserve(reserve)
+        before = c.scratch_bytes()
+        g = _capture(c, stream, lambda: w.matmul_batch_dev(X, m, Y, rows, cols))
+        assert c.scratch_bytes() == before
+        first = None
+        for _ in range(3):
+            Y.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            first = Y.clone() if first is None else first
+            assert torch.equal(Y, first) and torch.isfinite(Y).all()
+        w.matmul_batch_dev(X, m, Y, rows, cols)  # eager, with scratch
+        torch.cuda.synchronize()
+        if reserve:
+            assert torch.equal(Y, first)
+        else:
+            # fp32 sums in another order: both within 1e-5 sum|w x| of exact (test_gpu_parity)
+            bound = 2e-5 * float(abs(X).sum(1).max()) * float(abs(torch.from_numpy(w.dequant(0, rows * cols))).max())
+            assert float((Y - first).abs().max()) <= bound
+        w.free()
+    finally:
+        torch.cuda.synchronize()
+        c.close()

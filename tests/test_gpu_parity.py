@@ -988,3 +988,94 @@ def test_moe_route_edge_cases(g4, ctx, oracle, case):
         rids, rw = oracle.route(lg, K, renorm)
         assert np.array_equal(ids, rids), (case, renorm)
         assert same_bits(w, rw), (case, renorm)
+
+
+# Several tokens on the matrix cores (k_mat): per format the sizes at which its
+# tiles and slices have edges.  Rows that are not whole tiles, one to four blocks
+# in the last slice (columns 32, 64 and 96 past a multiple of 128), workgroups of
+# 4, 8 and 16 waves with slices to spare, column splits (2176 and 8192 columns),
+# rows behind an offset, one to three token tiles, and enough rows that a
+# workgroup walks several tiles.  BF16 and F16 take this route from three tokens
+# on, the others here from nine.
+MAT_SHAPES = [(9, 17, 512, 0), (16, 33, 1024, 1), (17, 40, 2048, 0), (33, 50, 1152, 2), (40, 24, 2176, 0),
+              (9, 20, 8192, 0), (64, 4500, 256, 0)]
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, Q5_K, Q6_K, BF16, F16])
+@pytest.mark.parametrize("m,rows,dim1,off_rows", MAT_SHAPES)
+def test_batched_matrix_core_shapes(g4, ctx, oracle, t, m, rows, dim1, off_rows):
+    _batched_case(g4, ctx, oracle, t, m, rows, dim1, off_rows)
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_0])
+@pytest.mark.parametrize("m,rows,dim1,off_rows", [(9, 20, 32, 0), (9, 35, 544, 1), (20, 18, 1056, 0), (11, 16, 2144, 3)])
+def test_batched_matrix_core_odd_blocks(g4, ctx, oracle, t, m, rows, dim1, off_rows):
+    _batched_case(g4, ctx, oracle, t, m, rows, dim1, off_rows)
+
+
+@pytest.mark.parametrize("t,m,rows,dim1", [(BF16, 3, 40, 64), (F16, 3, 33, 192), (BF16, 5, 20, 2112),
+                                           (Q8_0, 4, 8192, 1024), (Q4_0, 6, 2048, 4096), (Q6_K, 4, 4096, 2048)])
+def test_batched_matrix_core_few_tokens(g4, ctx, oracle, t, m, rows, dim1):
+    _batched_case(g4, ctx, oracle, t, m, rows, dim1, 0)
+
+
+def _no_subnormals(t, raw):
+    """F16 weights without subnormals: the vector path reads them as 0
+    (F16FloatTensor.kt:59-61), the exact sum does not."""
+    if t != F16:
+        return raw
+    raw = raw.copy()
+    h = raw.view(np.uint16)
+    h[(h & 0x7C00) == 0] = 0
+    return raw
+
+
+def _batched_case(g4, ctx, oracle, t, m, rows, dim1, off_rows):
+    announce("batched type %d M=%d rows=%d dim1=%d off_rows=%d" % (t, m, rows, dim1, off_rows))
+    n, off = -(-(rows + off_rows) * dim1 // 256) * 256, off_rows * dim1
+    raw = _no_subnormals(t, synth.weights(61, "mt%d.%d.%d" % (t, rows, dim1), t, n))
+    X = synth.activations(61, "mtx%d.%d" % (m, dim1), m * dim1).reshape(m, dim1)
+    w = upload(g4, ctx, t, raw, n)
+    Y = w.matmul_batch(X, rows, dim1, off)
+    for i in range(m):
+        ex, ab = oracle.matmul_exact(t, raw, X[i], rows, dim1, off)
+        assert_dots(Y[i], ex, ab, "token %d" % i)
+    w.free()
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, Q5_K, Q6_K, BF16, F16])
+def test_batched_matrix_core_non_finite_and_wide_x(g4, ctx, oracle, t):
+    """Infinite and NaN activations reach their own tokens' outputs as in the sum of
+    the products w * x (NaN for w = 0, else of the infinity's sign); a token spanning
+    1e-20..1e20 and the finite tokens that share the waves stay within the bound."""
+    announce("batched non-finite x type %d" % t)
+    m, rows, dim1 = 12, 40, 2048
+    raw = _no_subnormals(t, synth.weights(62, "mtn%d" % t, t, rows * dim1))
+    X = synth.activations(62, "mtnx", m * dim1).reshape(m, dim1)
+    X[4] *= (10.0 ** np.random.default_rng(62).uniform(-20, 20, dim1)).astype(np.float32)
+    X[1, 5], X[2, 700], X[3, dim1 - 7] = np.inf, np.nan, -np.inf
+    w = upload(g4, ctx, t, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    for i in range(m):
+        ex, ab = oracle.matmul_exact(t, raw, X[i], rows, dim1)
+        if i in (1, 2, 3):
+            assert not np.any(np.isfinite(Y[i]))
+            assert np.array_equal(np.isnan(Y[i]), np.isnan(ex)) and np.array_equal(Y[i] > 0, ex > 0)
+        else:
+            assert_dots(Y[i], ex, ab, "token %d" % i)
+    w.free()
+
+
+def test_batched_matrix_core_infinite_weight(g4, ctx, oracle):
+    """An infinite BF16 weight gives its row infinite outputs (not the NaN that an
+    infinity times an activation's zero residual part would)."""
+    announce("batched infinite bf16 weight")
+    m, rows, dim1 = 5, 20, 512
+    raw = synth.weights(63, "mti", BF16, rows * dim1).copy()
+    raw.view(np.uint16)[3 * dim1 + 100] = 0x7F80
+    X = np.ones((m, dim1), np.float32)
+    w = upload(g4, ctx, BF16, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    assert np.all(Y[:, 3] == np.inf)
+    assert np.all(np.isfinite(np.delete(Y, 3, 1)))
+    w.free()

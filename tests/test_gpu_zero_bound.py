@@ -191,3 +191,21 @@ def test_zero_down_experts_give_exact_zero(g4, ctx, oracle):
     assert np.all(Y2 == 0.0)
     wgu.free()
     wdn.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", [Q4_0, Q5_K])
+def test_zero_rows_batched_many(g4, ctx, oracle, t):
+    """20 tokens of the formats other than Q4_K take their own matrix-core kernel:
+    Q4_0's integers are 0 where the weight is, Q5_K's two sums run alike."""
+    announce("zero-bound batched type %d M=20" % t)
+    rows, cols, m = 96, 2048, 20
+    kinds = _kinds(rows)
+    raw = BUILD[t](rows, cols, kinds)
+    X = synth.activations(8, "X%d" % m, m * cols).reshape(m, cols)
+    w = g4.FloatTensorFactory.create(ctx, t, raw, rows * cols)
+    Y = w.matmul_batch(X, rows, cols)
+    for i in range(m):
+        y64, ab = oracle.matmul_exact(t, raw, X[i], rows, cols)
+        _check(Y[i], y64, ab, kinds, "batched token %d" % i)
+    w.free()
