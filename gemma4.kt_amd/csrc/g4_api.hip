@@ -497,10 +497,10 @@ int check_moe(g4_ctx *ctx, const g4_weight *wgu, const g4_weight *wdn, int32_t T
 // Routing done inside the gate+up launch (g4_moe_routed*): the router logits in,
 // the ids and weights it stores out.
 // Calls of at least this many tokens run the experts grouped (launch_moe_grp):
-// measured on the 128-expert top-8 shape (alternating runs, one box), the grouped
-// launches take 231, 233, 235, 239 and 288 us at 33, 40, 48, 64 and 128 tokens
-// against 201, 233, 275, 332 and 723 us for the per-pair ones, and about 222-230
-// us from 16 to 32 tokens, where the per-pair ones take 101-180 us.
+// measured on the 128-expert top-8 shape, the grouped launches take 174, 200, 213,
+// 220, 224, 226, 238 and 272 us at 16, 24, 32, 40, 48, 64, 128 and 200 tokens, the
+// per-pair ones 107, 151, 177 and 223 us at 16, 24, 32 and 40, 332 at 64 and 723 at
+// 128.
 constexpr int32_t MOE_GROUPED_MIN_T = 41;
 
 struct MoeRoute {
@@ -553,7 +553,7 @@ int moe_dev(g4_ctx *ctx, const g4_weight *wgu, const g4_weight *wdn, int32_t n_e
     dn.x_div = 1;
     dn.y = d_ys;
     dn.y_stride = dim;
-    if (g4::moe_grp_ok(wgu->type, gu) && g4::moe_grp_ok(wdn->type, dn) && n_experts < 65535 &&
+    if (g4::moe_grp_ok(wgu->type, true, gu) && g4::moe_grp_ok(wdn->type, false, dn) && n_experts < 65535 &&
         (!route || route->n_experts <= g4::ROUTE_LAUNCH_MAX_E)) {
       if (route)
         G4_TRY(launch_status(g4::launch_route(route->d_logits, T, route->n_experts, k, route->renormalize,

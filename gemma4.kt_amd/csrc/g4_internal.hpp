@@ -134,7 +134,7 @@ struct MoeGrpArgs {
   // before gelu (the 16-pair tiles write them here, then k_gelu_mul forms y)
   float *gu;
 };
-bool moe_grp_ok(int type, const MoeGrpArgs &a);
+bool moe_grp_ok(int type, bool gate_up, const MoeGrpArgs &a);
 // Grants the grouped kernels their largest dynamic LDS size on the current
 // device; called once per device before any launch (g4_open).
 hipError_t moe_grp_init_device();

@@ -935,21 +935,25 @@ __global__ __launch_bounds__(MG_WPB * 64) void k_moe_grp(MoeGrpArgs a) {
 }
 
 // -------------------------------------------- grouped MoE, 16-pair tiles ----
-// The experts of a multi-token MoE call on k_tok_q4k's tiles.  Workgroup (row
-// block, expert e) takes e's (token, slot) pairs sixteen at a time in pair order
-// (a pass): pair slot t is MFMA row t, its token's x split into bf16 parts in the
-// waves' registers as a 16-token tile (wave w: columns 128 w .. 128 w + 127), and
-// the workgroup walks its 16-row tiles with the 16 q weight operands, each weight
+// The experts of a multi-token MoE call on k_tok_q4k's tiles.  Each expert's
+// (token, slot) pairs are taken sixteen at a time in pair order (a pass): pair
+// slot t is MFMA row t, its token's x split into bf16 parts in the waves'
+// registers as a 16-token tile (wave w: columns 128 w .. 128 w + 127), and the
+// expert's 16-row tiles are walked with the 16 q weight operands, each weight
 // read once per pass.  Row r of pair p goes to y[p * y_stride + r]; the gate+up
 // launch runs the expert's gate and up rows as one matrix of 2 ff rows (its two
-// halves adjacent in the slab) and k_gelu_mul forms h.  Workgroups (x,
-// n_experts) write the zero rows of pairs whose id is out of range.  Rows of up
-// to 2048 columns: one column split, no partial sums.
+// halves adjacent in the slab) and k_gelu_mul forms h.  Rows of up to 2048
+// columns: one column split, no partial sums.
+//
+// Work split: the passes of all experts, counted by every workgroup from the ids,
+// times their row tiles are one sequence of units, and each of the CU-many
+// workgroups takes an equal stretch of it, whatever the routing: at most two or
+// three passes' x, and no CU waits for an expert with twice the pairs.  (Row blocks
+// x experts, each looping over its passes, left most CUs idle while the experts of
+// more than 16 pairs ran their second pass: 200 tokens, 128 experts, top-8,
+// 429 -> 271 us a call; 60 tokens, 32 experts, top-4, ff 704, 117 -> 71 us.)
 constexpr int GT_WPB = 16;
-// row blocks per expert: this many per CU share of the experts (with 128 experts
-// on 256 CUs, two; measured at 128 tokens equal with four, at 40-64 tokens 7%
-// faster than four and 8-20% faster than eight)
-constexpr int GT_GX_PER_CU = 1;
+constexpr int GT_MAX_E = GT_WPB * 64;  // experts: one thread each
 
 template <bool AL>
 __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
@@ -961,7 +965,9 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
       lds[RED_BYTES + WST_BYTES > XST_BYTES ? RED_BYTES + WST_BYTES : XST_BYTES];
   __shared__ int pl[16];      // the pass's pairs (-1: none)
   __shared__ int tl[16];      // their tokens (empty slots: the first pair's)
-  __shared__ int wcnt[WPB];   // matches per wave in a scan step
+  __shared__ int wcnt[WPB];   // matches per wave in a scan step; passes per wave of experts
+  __shared__ int ecnt[GT_MAX_E + 1];  // pairs per expert, and pairs of no expert
+  __shared__ int cur[2];      // the current unit's expert and pass
   f32x4(*red)[WPB][64] = (f32x4(*)[WPB][64])lds;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -969,26 +975,48 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
   const int C = a.dim1 >> 6;
   const int g0 = wid * GPW;                     // first group of this wave's slice (even)
   const int ng = max(0, min(GPW, C - g0));      // wave-uniform
-  const int e = blockIdx.y;
-  const bool zero_rows = e == a.n_experts;
   const int n_rt = (a.rows + 15) >> 4;
-  const int rpb = (n_rt + gridDim.x - 1) / gridDim.x;
-  const int rt0 = min(n_rt, (int)blockIdx.x * rpb), rt1 = min(n_rt, rt0 + rpb);
-  if (rt0 >= rt1) return;  // the whole workgroup
-  const int64_t base = (zero_rows ? 0 : (int64_t)e * a.expert_stride) + a.base0;
 
-  // pairs of rank 16 pass .. 16 pass + 15 among this expert's into pl; returns
-  // the number of its pairs (the same in every thread)
-  auto scan = [&](int pass) {
+  // passes of expert tid, and those before it
+  for (int k = tid; k <= a.n_experts; k += WPB * 64) ecnt[k] = 0;
+  __syncthreads();
+  for (int p = tid; p < a.S; p += WPB * 64) {
+    const int id = a.ids[p];
+    atomicAdd(&ecnt[id >= 0 && id < a.n_experts ? id : a.n_experts], 1);
+  }
+  __syncthreads();
+  const int np = tid < a.n_experts ? (ecnt[tid] + 15) >> 4 : 0;
+  int before = np;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int v = __shfl_up(before, d, 64);
+    before += lane >= d ? v : 0;
+  }
+  if (lane == 63) wcnt[wid] = before;
+  __syncthreads();
+  int all = 0;
+#pragma unroll
+  for (int w = 0; w < WPB; ++w) {
+    before += w < wid ? wcnt[w] : 0;
+    all += wcnt[w];
+  }
+  const bool none = ecnt[a.n_experts] > 0;  // some pairs have no expert: their rows are zeros
+  __syncthreads();  // ecnt and wcnt are reused
+  if (tid < a.n_experts) ecnt[tid] = (before - np) << 13 | np;  // at most 4096 passes (MG_MAX_S)
+  if (none)
+    for (int p = blockIdx.x; p < a.S; p += gridDim.x) {
+      const int id = a.ids[p];
+      if (id >= 0 && id < a.n_experts) continue;
+      for (int r = tid; r < a.rows; r += WPB * 64) a.y[(int64_t)p * a.y_stride + r] = 0.f;
+    }
+
+  // pairs of rank 16 pass .. 16 pass + 15 among expert e's into pl
+  auto scan = [&](int e, int pass) {
     if (tid < 16) pl[tid] = -1;
     int total = 0;
-    for (int p0 = 0; p0 < a.S; p0 += WPB * 64) {
+    for (int p0 = 0; p0 < a.S && total < 16 * (pass + 1); p0 += WPB * 64) {
       const int p = p0 + tid;
-      bool m = false;
-      if (p < a.S) {
-        const int id = a.ids[p];
-        m = zero_rows ? (id < 0 || id >= a.n_experts) : id == e;
-      }
+      const bool m = p < a.S && a.ids[p] == e;
       const uint64_t b = __builtin_amdgcn_ballot_w64(m);
       if (lane == 0) wcnt[wid] = __builtin_popcountll(b);
       __syncthreads();
@@ -1006,68 +1034,83 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
     }
     if (tid < 16) tl[tid] = (pl[tid] >= 0 ? pl[tid] : pl[0]) / a.x_div;
     __syncthreads();
-    return total;
   };
 
-  const int64_t w_step = (16 * a.row_stride >> 8) * 144;  // 16 rows: whole super-blocks
-  // weight group gi of row tile rt, this lane's row (B column n) and K-slice j
-  auto load_w = [&](int rt, bool live, u32x2a4 (&Q)[GPW], u32x4 (&H)[NH], int (&gs)[GPW]) {
-    const int r = rt * 16 + n;
-    const bool rok = live && r < a.rows;
-#pragma unroll
-    for (int gi = 0; gi < GPW; ++gi) {
-      // rows past the end and groups past the slice read the first group of
-      // the tensor (in bounds; never stored / never multiplied)
-      const int64_t el = (rok && gi < ng) ? base + (int64_t)r * a.row_stride + (int64_t)(g0 + gi) * 64 : 0;
-      const int64_t G = el >> 6;
-      const uint8_t *sb = a.W + (G >> 2) * 144;
-      gs[gi] = (int)(G & 3);
-      H[gi] = *(const u32x4 *)sb;
-      Q[gi] = *(const u32x2a4 *)(sb + 16 + 32 * (G & 3) + 8 * j);
+  // The stretch [u, u1) of units.  With fewer passes than workgroups, one pass (or
+  // a part of one) per workgroup where the longest part is no longer than an equal
+  // stretch and the start of the second pass in it (about five tiles' time: its
+  // pairs, their x and its split).
+  const int64_t units = (int64_t)all * n_rt;
+  const int parts = all > 0 ? (int)gridDim.x / all : 0, bx = (int)blockIdx.x;
+  int64_t u = units * bx / (int)gridDim.x, u1 = units * (bx + 1) / (int)gridDim.x;
+  if (parts > 0) {
+    const int len = (n_rt + parts - 1) / parts;
+    if (len <= units / (int)gridDim.x + 5) {
+      const int item = bx / parts, t0 = min(n_rt, bx % parts * len);
+      u = item < all ? (int64_t)item * n_rt + t0 : 0;
+      u1 = item < all ? (int64_t)item * n_rt + min(n_rt, t0 + len) : 0;
     }
-  };
-  // AL: a tile's 16 rows x (head + the wave's two groups) read by four adjacent
-  // lanes per row and staged in the wave's own LDS rows (as k_tok_q4k does).
-  // Rows start on a group pair (row_stride a multiple of 128: the MoE down
-  // rows of 1408 columns start every second one half way into a super-block),
-  // so a wave's two groups lie in one super-block, at a row-dependent position
-  // that repeats every 16 rows (16 rows are whole super-blocks)
-  unsigned char *wst = lds + RED_BYTES + (size_t)wid * 16 * WROW;
-  const int64_t e_st = base + (int64_t)(rt0 * 16 + (lane >> 2)) * a.row_stride + (int64_t)g0 * 64;
-  const uint8_t *w_tile0 = a.W + (e_st >> 8) * 144;
-  const int q_st = 16 + 32 * (int)((e_st >> 6) & 3) + 16 * (lane & 3);
-  // which half of its super-block row n's groups are in (the scales' byte positions)
-  const int hq_n = (int)((((int64_t)n * a.row_stride + (int64_t)g0 * 64 + base) >> 7) & 1);
-  auto load_raw = [&](int rt, bool live, u32x4 &QR, uint32_t &HR) {
-    // rows past the end read the tensor's first super-block
-    const bool ok = live && ng > 0 && rt * 16 + (lane >> 2) < a.rows;
-    const uint8_t *sb = ok ? w_tile0 + (int64_t)(rt - rt0) * w_step : a.W;
-    QR = *(const u32x4 *)(sb + (ok ? q_st : 16));
-    HR = *(const uint32_t *)(sb + 4 * (lane & 3));
-  };
-  auto stage = [&](const u32x4 &QR, uint32_t HR, u32x2a4 (&Q)[GPW], u32x4 (&H)[NH]) {
-    unsigned char *wr = wst + (lane >> 2) * WROW;
-    *(u32x4 *)(wr + 16 + 16 * (lane & 3)) = QR;
-    *(uint32_t *)(wr + 4 * (lane & 3)) = HR;
-    const unsigned char *rd = wst + n * WROW;
-    H[0] = *(const u32x4 *)rd;
-#pragma unroll
-    for (int gi = 0; gi < GPW; ++gi) Q[gi] = *(const u32x2a4 *)(rd + 16 + 32 * gi + 8 * j);
-  };
+  }
+  while (u < u1) {
+    const int item = (int)(u / n_rt), rt0 = (int)(u - (int64_t)item * n_rt);
+    const int rt1 = (int)min((int64_t)n_rt, rt0 + (u1 - u));
+    u += rt1 - rt0;
+    __syncthreads();  // every wave is done with the previous pass's LDS
+    if (tid < a.n_experts) {
+      const int k = item - (ecnt[tid] >> 13);
+      if (k >= 0 && k < (ecnt[tid] & 0x1FFF)) cur[0] = tid, cur[1] = k;
+    }
+    __syncthreads();
+    const int e = __builtin_amdgcn_readfirstlane(cur[0]);
+    scan(e, __builtin_amdgcn_readfirstlane(cur[1]));
+    const int64_t base = (int64_t)e * a.expert_stride + a.base0;
 
-  for (int pass = 0;; ++pass) {
-    if (pass > 0) __syncthreads();  // every wave is done with the previous pass's LDS
-    const int total = scan(pass);
-    const int cnt = min(16, total - 16 * pass);
-    if (cnt <= 0) return;
-    if (zero_rows) {
-      const int r0 = rt0 * 16, nr = min(a.rows, rt1 * 16) - r0;
-      for (int i = tid; i < cnt * nr; i += WPB * 64) {
-        const int t = i / nr, r = r0 + i % nr;
-        a.y[(int64_t)pl[t] * a.y_stride + r] = 0.f;
+    const int64_t w_step = (16 * a.row_stride >> 8) * 144;  // 16 rows: whole super-blocks
+    // weight group gi of row tile rt, this lane's row (B column n) and K-slice j
+    auto load_w = [&](int rt, bool live, u32x2a4 (&Q)[GPW], u32x4 (&H)[NH], int (&gs)[GPW]) {
+      const int r = rt * 16 + n;
+      const bool rok = live && r < a.rows;
+#pragma unroll
+      for (int gi = 0; gi < GPW; ++gi) {
+        // rows past the end and groups past the slice read the first group of
+        // the tensor (in bounds; never stored / never multiplied)
+        const int64_t el = (rok && gi < ng) ? base + (int64_t)r * a.row_stride + (int64_t)(g0 + gi) * 64 : 0;
+        const int64_t G = el >> 6;
+        const uint8_t *sb = a.W + (G >> 2) * 144;
+        gs[gi] = (int)(G & 3);
+        H[gi] = *(const u32x4 *)sb;
+        Q[gi] = *(const u32x2a4 *)(sb + 16 + 32 * (G & 3) + 8 * j);
       }
-      continue;
-    }
+    };
+    // AL: a tile's 16 rows x (head + the wave's two groups) read by four adjacent
+    // lanes per row and staged in the wave's own LDS rows (as k_tok_q4k does).
+    // Rows start on a group pair (row_stride a multiple of 128: the MoE down
+    // rows of 1408 columns start every second one half way into a super-block),
+    // so a wave's two groups lie in one super-block, at a row-dependent position
+    // that repeats every 16 rows (16 rows are whole super-blocks)
+    unsigned char *wst = lds + RED_BYTES + (size_t)wid * 16 * WROW;
+    const int64_t e_st = base + (int64_t)(rt0 * 16 + (lane >> 2)) * a.row_stride + (int64_t)g0 * 64;
+    const uint8_t *w_tile0 = a.W + (e_st >> 8) * 144;
+    const int q_st = 16 + 32 * (int)((e_st >> 6) & 3) + 16 * (lane & 3);
+    // which half of its super-block row n's groups are in (the scales' byte positions)
+    const int hq_n = (int)((((int64_t)n * a.row_stride + (int64_t)g0 * 64 + base) >> 7) & 1);
+    auto load_raw = [&](int rt, bool live, u32x4 &QR, uint32_t &HR) {
+      // rows past the end read the tensor's first super-block
+      const bool ok = live && ng > 0 && rt * 16 + (lane >> 2) < a.rows;
+      const uint8_t *sb = ok ? w_tile0 + (int64_t)(rt - rt0) * w_step : a.W;
+      QR = *(const u32x4 *)(sb + (ok ? q_st : 16));
+      HR = *(const uint32_t *)(sb + 4 * (lane & 3));
+    };
+    auto stage = [&](const u32x4 &QR, uint32_t HR, u32x2a4 (&Q)[GPW], u32x4 (&H)[NH]) {
+      unsigned char *wr = wst + (lane >> 2) * WROW;
+      *(u32x4 *)(wr + 16 + 16 * (lane & 3)) = QR;
+      *(uint32_t *)(wr + 4 * (lane & 3)) = HR;
+      const unsigned char *rd = wst + n * WROW;
+      H[0] = *(const u32x4 *)rd;
+#pragma unroll
+      for (int gi = 0; gi < GPW; ++gi) Q[gi] = *(const u32x2a4 *)(rd + 16 + 32 * gi + 8 * j);
+    };
+
     // the pair of the outputs this lane stores (component wid of its four, waves 0..3)
     const int pj = pl[4 * j + (wid & 3)];
 
@@ -1271,18 +1314,20 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
 // True when the 16-pair tiles take a grouped launch: Q4_K rows of at most 2048
 // columns in 64-column groups; the gate+up launch's gate and up halves adjacent.
 static bool grp_tok_ok(bool gate_up, const MoeGrpArgs &a) {
+  if (a.n_experts > GT_MAX_E) return false;
   if (a.dim1 <= 0 || a.dim1 > GT_WPB * TOK_GPW * 64 || a.dim1 % 64 != 0) return false;
   if (a.base0 % 64 != 0 || a.row_stride % 64 != 0 || a.expert_stride % 64 != 0) return false;
   if (gate_up && (a.gu == nullptr || a.base1 != a.base0 + (int64_t)a.rows * a.row_stride)) return false;
   return a.S >= 1 && a.rows >= 1 && a.x_div >= 1 && a.n_experts >= 1;
 }
 
-bool moe_grp_ok(int type, const MoeGrpArgs &a) {
-  if (type != T_Q4_K) return false;
+bool moe_grp_ok(int type, bool gate_up, const MoeGrpArgs &a) {
+  if (type != T_Q4_K || a.S > MG_MAX_S) return false;
+  if (grp_tok_ok(gate_up, a)) return true;
   if (a.dim1 <= 0 || a.dim1 % 128 != 0 || a.dim1 > MG_MAX_DIM1) return false;
   if (a.base0 % 128 != 0 || a.base1 % 128 != 0 || a.row_stride % 128 != 0 || a.expert_stride % 128 != 0)
     return false;
-  return a.S >= 1 && a.S <= MG_MAX_S && a.rows >= 1 && a.x_div >= 1 && a.n_experts >= 1;
+  return a.S >= 1 && a.rows >= 1 && a.x_div >= 1 && a.n_experts >= 1;
 }
 
 hipError_t moe_grp_init_device() {
@@ -1294,20 +1339,17 @@ hipError_t moe_grp_init_device() {
 }
 
 hipError_t launch_moe_grp(int type, bool gate_up, const MoeGrpArgs &a, const DevInfo &dev, hipStream_t s) {
-  if (!moe_grp_ok(type, a)) return hipErrorNotSupported;
+  if (!moe_grp_ok(type, gate_up, a)) return hipErrorNotSupported;
   if (grp_tok_ok(gate_up, a)) {
     // 16-pair tiles: the gate+up launch writes the gate and up rows (2 rows per
-    // pair) and k_gelu_mul forms h; row blocks per expert so that the experts'
-    // workgroups about fill the CUs
+    // pair) and k_gelu_mul forms h
     MoeGrpArgs b = a;
     if (gate_up) {
       b.rows = 2 * a.rows;
       b.y = a.gu;
       b.y_stride = 2 * (int64_t)a.rows;
     }
-    const int n_rt = (b.rows + 15) / 16;
-    const int gx = std::max(1, std::min(n_rt, GT_GX_PER_CU * dev.cu_count / std::max(1, b.n_experts)));
-    const dim3 grid((unsigned)gx, (unsigned)b.n_experts + 1);
+    const dim3 grid((unsigned)dev.cu_count);
     // rows starting on a group pair and whole 128-column slices: the coalesced,
     // LDS-staged weight tiles
     const bool al = b.base0 % 128 == 0 && b.row_stride % 128 == 0 && b.expert_stride % 128 == 0 && b.dim1 % 128 == 0;

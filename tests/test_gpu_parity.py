@@ -1079,3 +1079,42 @@ def test_batched_matrix_core_infinite_weight(g4, ctx, oracle):
     assert np.all(Y[:, 3] == np.inf)
     assert np.all(np.isfinite(np.delete(Y, 3, 1)))
     w.free()
+
+
+# The grouped launches share the passes' row tiles out evenly over the CUs:
+# more passes than workgroups (300 experts, some hit twice over), a pass shared by
+# several (one expert: its 24 tiles on as many workgroups), stretches that end
+# within a pass (90 passes over 256 CUs) and span two, an expert with most of the
+# pairs, pairs of no expert, and down rows that start on a 64-column group (320).
+@pytest.mark.parametrize("E,D,FF,K,T,skew,drop", [(300, 256, 128, 8, 120, 0, 0), (1, 512, 192, 1, 50, 0, 0),
+                                                   (90, 256, 320, 2, 60, 0, 0), (24, 256, 128, 4, 100, 60, 7),
+                                                   (16, 128, 64, 2, 45, 0, 45)])
+def test_moe_grouped_equal_stretches(g4, ctx, oracle, E, D, FF, K, T, skew, drop):
+    announce("moe grouped stretches E=%d D=%d FF=%d K=%d T=%d" % (E, D, FF, K, T))
+    gu = synth.q4_k(66, "gu%d.%d" % (E, FF), E * 2 * FF * D)
+    dn = synth.q4_k(66, "dn%d.%d" % (E, FF), E * D * FF)
+    X = synth.activations(66, "X%d" % T, T * D).reshape(T, D)
+    rng = np.random.default_rng(66)
+    ids = np.stack([rng.permutation(E)[:K] for _ in range(T)]).astype(np.int32)
+    ids[:skew, 0] = 5 % E
+    w = rng.uniform(0.1, 1.0, (T, K)).astype(np.float32)
+    gone = np.zeros((T, K), bool)
+    gone.reshape(-1)[rng.permutation(T * K)[:drop]] = True
+    bad = ids.copy()
+    bad[gone] = np.where(np.arange(int(gone.sum())) % 2, E, -1)
+    wgu = upload(g4, ctx, Q4_K, gu, E * 2 * FF * D)
+    wdn = upload(g4, ctx, Q4_K, dn, E * D * FF)
+    import torch
+    d_Y = torch.empty((T, D), device="cuda")
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        g4.moe_dev(ctx, wgu, wdn, torch.from_numpy(X).cuda(), T, D, FF, torch.from_numpy(bad).cuda(),
+                   torch.from_numpy(w).cuda(), K, d_Y)
+        torch.cuda.synchronize()
+    finally:
+        ctx.set_stream(None)
+    Y = d_Y.cpu().numpy()
+    y64, bound = oracle.moe_exact(Q4_K, gu, Q4_K, dn, X, ids, np.where(gone, 0.0, w).astype(np.float32), D, FF)
+    assert_dots(Y.reshape(-1), y64.reshape(-1), bound.reshape(-1), "grouped stretches")
+    wgu.free()
+    wdn.free()
