@@ -8,7 +8,7 @@
 //
 // Work split, as k_tok_q4k's: a wave keeps 16 tokens x 128 columns of x split in
 // registers and walks the workgroup's 16-row tiles; the waves of a workgroup take
-// adjacent columns, and their partial tiles are summed in wave order through LDS
+// adjacent columns, and their partial tiles are summed through LDS in a fixed order
 // (deterministic).  More tokens are further workgroups, which share a row block's
 // weights through the L2.  Rows of more than 2048 columns split over workgroups,
 // whose partial sums launch_tok_reduce adds in order.
@@ -255,6 +255,9 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
             P[b][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[b][p], B[b], P[b][0], 0, 0, 0);
           }
         }
+      if constexpr (HALF)
+        acc = (P[0][0] + P[1][0]) + (P[2][0] + P[3][0]);
+      else
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         f32x4 S;
@@ -268,8 +271,6 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
             acc[i] += rounded(sc[0][b] * P[b][0][i]) - rounded(of[b] * S[i]);
           } else if constexpr (SPB == 1) {
             acc[i] = __builtin_fmaf(sc[0][b], P[b][0][i], acc[i]);
-          } else {
-            acc[i] += P[b][0][i];
           }
         }
       }
@@ -277,12 +278,18 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
     red[buf][wid][lane] = acc;
     put(wr);
     __syncthreads();
-    // the slices summed in wave order: wave c takes component c of every lane's four
+    // the slices summed pairwise (fewer roundings than one after the other): wave c
+    // takes component c of every lane's four
     if (wid < 4) {
       const float *rp = (const float *)&red[buf][0][lane] + wid;
-      float s = rp[0];
+      float v[WPB];
 #pragma unroll
-      for (int w = 1; w < WPB; ++w) s += rp[w * 64 * 4];
+      for (int w = 0; w < WPB; ++w) v[w] = rp[w * 64 * 4];
+#pragma unroll
+      for (int d = WPB / 2; d >= 1; d >>= 1)
+#pragma unroll
+        for (int w = 0; w < d; ++w) v[w] = v[2 * w] + v[2 * w + 1];
+      float s = v[0];
       const int r = rt * 16 + n, m = 4 * j + wid;
       if (r < a.rows && m < mt) {
         if (s != s)
