@@ -50,6 +50,14 @@ struct g4_ctx {
   size_t pin_used;
   G4PendingOut outs[8];
   int n_outs;
+  // Workspace of the tiled many-token product (grow-only), apart from `scratch`:
+  // calls that are not being captured use it, so no graph holds its address, and
+  // mm_acquire orders calls on different streams over it.
+  char *mm_ws;
+  size_t mm_bytes;
+  bool mm_used;           // queued work may still use it,
+  hipStream_t mm_stream;  // the last of it on this stream,
+  hipEvent_t mm_event;    // and ended by this event once calls have come on a second stream (else null)
 };
 
 struct g4_weight {
@@ -185,6 +193,67 @@ int ensure_scratch(g4_ctx *ctx, size_t bytes) {
 // is avoided: the degenerate shapes below may run under capture).
 int zero_dev(g4_ctx *ctx, void *p, size_t bytes) {
   G4_HIP(g4::launch_zero(p, bytes, ctx->stream), "zero fill");
+  return G4_OK;
+}
+
+// The tiled product's workspace of `bytes`, safe to use by work queued on the
+// context's stream from here on; null when the call has to do without: its
+// stream is being captured, the stream of the last use is, or no memory is left.
+// Calls on one stream need no ordering.  The first use on a second stream waits
+// for the last one on the host; from then on every use records an event and a
+// change of stream waits for it on the GPU.
+char *mm_acquire(g4_ctx *ctx, size_t bytes) {
+  if (ctx->capturing) return nullptr;
+  const bool grow = bytes > ctx->mm_bytes, moved = ctx->mm_used && ctx->mm_stream != ctx->stream;
+  if (!grow && !moved) return ctx->mm_ws;
+  if (!grow && ctx->mm_event) {
+    if (hipStreamWaitEvent(ctx->stream, ctx->mm_event, 0) == hipSuccess) return ctx->mm_ws;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  // another thread's capture is not disturbed by the allocation and the waits
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+  bool ok = true;
+  if (ctx->mm_used) {
+    if (ctx->mm_event) {
+      ok = hipEventSynchronize(ctx->mm_event) == hipSuccess;
+    } else {
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(ctx->mm_stream, &st) != hipSuccess)
+        ok = hipDeviceSynchronize() == hipSuccess;  // the stream is gone
+      else
+        ok = st == hipStreamCaptureStatusNone && hipStreamSynchronize(ctx->mm_stream) == hipSuccess;
+    }
+    if (ok) ctx->mm_used = false;
+  }
+  if (ok && moved && !ctx->mm_event && hipEventCreateWithFlags(&ctx->mm_event, hipEventDisableTiming) != hipSuccess) {
+    ctx->mm_event = nullptr;
+    ok = false;
+  }
+  if (ok && grow) {
+    if (ctx->mm_ws) (void)hipFree(ctx->mm_ws);
+    ctx->mm_ws = nullptr;
+    ctx->mm_bytes = 0;
+    const size_t want = std::max(bytes, size_t(64) << 20);
+    void *p = nullptr;
+    if (hipMalloc(&p, want) == hipSuccess) {
+      ctx->mm_ws = (char *)p;
+      ctx->mm_bytes = want;
+    } else {
+      ok = false;
+    }
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (!ok) (void)hipGetLastError();  // the caller takes another route
+  return ok ? ctx->mm_ws : nullptr;
+}
+
+// The workspace's use is queued on the context's stream.
+int mm_release(g4_ctx *ctx) {
+  ctx->mm_used = true;
+  ctx->mm_stream = ctx->stream;
+  if (ctx->mm_event) G4_HIP(hipEventRecord(ctx->mm_event, ctx->stream), "hipEventRecord");
   return G4_OK;
 }
 
@@ -379,24 +448,27 @@ g4::TokArgs tok_args(const g4_weight *w, int64_t off, const float *d_X, int32_t 
 
 // How a batched call runs, and the scratch floats it needs for partial sums.
 struct BatchRoute {
-  enum Kind { ROWS, TOK, MAT } kind;
+  enum Kind { ROWS, TOK, MAT, MM } kind;
   int64_t part;
+  char *ws;  // MM: the tiled product's workspace
 };
 
 // Several tokens of one matrix: the matrix-core kernels unpack each weight once
-// for 16 of them (Q4_K: g4_tok.hip, the other formats: g4_mat.hip); the row engine
-// runs one segment per token.
-BatchRoute batch_route(const g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1) {
-  if (M < 3 || dim0 == 0 || dim1 == 0) return {BatchRoute::ROWS, 0};
+// for 16 of them (Q4_K: g4_tok.hip, the other formats: g4_mat.hip), or for 128
+// (g4_mm.hip) where there is a workspace; the row engine runs one segment per token.
+BatchRoute batch_route(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1) {
+  if (M < 3 || dim0 == 0 || dim1 == 0) return {BatchRoute::ROWS, 0, nullptr};
   const g4::TokArgs t = tok_args(w, off, nullptr, M, nullptr, dim0, dim1);
+  if (g4::mm_ok(w->type, t, ctx->dev))
+    if (char *ws = mm_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))) return {BatchRoute::MM, 0, ws};
   // Two tokens stay on the row engine: measured on 8192 x 2048 Q4_K, 6.5 us against
   // 8.9 us for the matrix cores; from three on the matrix cores are as fast or
   // faster (9.1 / 9.3 us at M = 3, 9.6 / 14.4 at M = 8).  For the other formats
   // mat_min_tokens draws the line.
-  if (g4::tok_ok(w->type, t)) return {BatchRoute::TOK, g4::tok_scratch_floats(t, ctx->dev)};
+  if (g4::tok_ok(w->type, t)) return {BatchRoute::TOK, g4::tok_scratch_floats(t, ctx->dev), nullptr};
   if (M >= g4::mat_min_tokens(w->type, t) && g4::mat_ok(w->type, t))
-    return {BatchRoute::MAT, g4::mat_scratch_floats(t, ctx->dev)};
-  return {BatchRoute::ROWS, 0};
+    return {BatchRoute::MAT, g4::mat_scratch_floats(t, ctx->dev), nullptr};
+  return {BatchRoute::ROWS, 0, nullptr};
 }
 
 // The route of a call that needs `before` bytes of scratch besides, with that
@@ -408,7 +480,7 @@ int batch_prepare(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32
   *r = batch_route(ctx, w, off, M, dim0, dim1);
   const int rc = ensure_scratch(ctx, before + sizeof(float) * (size_t)r->part);
   if (rc == G4_OK || r->kind != BatchRoute::MAT || r->part == 0) return rc;
-  *r = {BatchRoute::ROWS, 0};
+  *r = {BatchRoute::ROWS, 0, nullptr};
   return ensure_scratch(ctx, before);
 }
 
@@ -418,6 +490,11 @@ int batch_dev(g4_ctx *ctx, const g4_weight *w, int64_t off, const float *d_X, in
   if (dim1 == 0) {
     G4_TRY(zero_dev(ctx, d_Y, sizeof(float) * (size_t)dim0 * M));
     return G4_OK;
+  }
+  if (r.kind == BatchRoute::MM) {
+    const hipError_t e = g4::launch_mm(w->type, tok_args(w, off, d_X, M, d_Y, dim0, dim1), r.ws, ctx->dev, ctx->stream);
+    G4_TRY(mm_release(ctx));
+    return launch_status(e, "matmul_batch");
   }
   if (r.kind != BatchRoute::ROWS) {
     g4::TokArgs t = tok_args(w, off, d_X, M, d_Y, dim0, dim1);
@@ -854,6 +931,11 @@ int g4_close(g4_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   (void)hipStreamSynchronize(ctx->own_stream);
+  if (ctx->mm_event) {
+    (void)hipEventSynchronize(ctx->mm_event);
+    (void)hipEventDestroy(ctx->mm_event);
+  }
+  if (ctx->mm_ws) (void)hipFree(ctx->mm_ws);
   if (ctx->scratch) (void)hipFree(ctx->scratch);
   for (int i = 0; i < ctx->n_retired; ++i) (void)hipFree(ctx->retired[i]);
   if (ctx->am_val) (void)hipFree(ctx->am_val);

@@ -107,6 +107,13 @@ int32_t mat_min_tokens(int type, const TokArgs &a);
 int64_t mat_scratch_floats(const TokArgs &a, const DevInfo &dev);
 hipError_t launch_mat(int type, const TokArgs &a, const DevInfo &dev, hipStream_t stream);
 
+// Many-token matmul on tiles of 128 tokens (g4_mm.hip; TokArgs::part is not used):
+// needs mm_ws_bytes() of 256-byte aligned workspace.  mm_ok: the type and offsets
+// take it and for these sizes it is the faster route.
+bool mm_ok(int type, const TokArgs &a, const DevInfo &dev);
+size_t mm_ws_bytes(int type, const TokArgs &a, const DevInfo &dev);
+hipError_t launch_mm(int type, const TokArgs &a, void *ws, const DevInfo &dev, hipStream_t stream);
+
 // Routed experts of a multi-token MoE call on the matrix cores, grouped by
 // expert (Q4_K): pair p = (token p / x_div, slot p % x_div) with expert ids[p]
 // reads x + (p / x_div) * x_stride and writes y + p * y_stride.  gate_up: rows

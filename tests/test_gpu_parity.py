@@ -1118,3 +1118,90 @@ def test_moe_grouped_equal_stretches(g4, ctx, oracle, E, D, FF, K, T, skew, drop
     assert_dots(Y.reshape(-1), y64.reshape(-1), bound.reshape(-1), "grouped stretches")
     wgu.free()
     wdn.free()
+
+
+# Many tokens in tiles of 128 (k_mm; rows and columns large enough that it is the
+# faster route): rows that are not whole tiles of 128, one to three token tiles
+# with a partial last one, an odd number of 64-column stages and a last one of 32
+# columns (Q8_0, Q4_0), column splits, rows behind an offset.
+@pytest.mark.parametrize("t,m,rows,dim1,off_rows", [
+    (Q8_0, 130, 4100, 2112, 0), (Q8_0, 201, 2050, 4128, 1), (Q4_0, 300, 4000, 2080, 0), (Q4_K, 512, 8200, 2048, 0),
+    (Q4_K, 500, 2500, 4160, 1), (Q6_K, 129, 4099, 2048, 0), (Q6_K, 257, 2048, 2368, 2), (F16, 150, 4098, 2048, 0),
+    (F16, 257, 3000, 1088, 1)])
+def test_batched_many_tokens_shapes(g4, ctx, oracle, t, m, rows, dim1, off_rows):
+    announce("batched many type %d M=%d rows=%d dim1=%d off_rows=%d" % (t, m, rows, dim1, off_rows))
+    n, off = -(-(rows + off_rows) * dim1 // 256) * 256, off_rows * dim1
+    raw = _no_subnormals(t, synth.weights(67, "mm%d.%d" % (t, dim1), t, n))
+    X = synth.activations(67, "mmx%d.%d" % (m, dim1), m * dim1).reshape(m, dim1)
+    w = upload(g4, ctx, t, raw, n)
+    Y = w.matmul_batch(X, rows, dim1, off)
+    for i in (0, 1, 31, 32, 63, 64, 95, 127, 128, m - 2, m - 1):
+        ex, ab = oracle.matmul_exact(t, raw, X[i], rows, dim1, off)
+        assert_dots(Y[i], ex, ab, "token %d" % i)
+    # every token: the same sums in another order (the tiles of 16 tokens)
+    for m0 in range(0, m, 48):
+        P = w.matmul_batch(X[m0:m0 + 48], rows, dim1, off)
+        scale = np.abs(P).max()
+        assert np.abs(P - Y[m0:m0 + 48]).max() <= 1e-5 * scale, m0
+    w.free()
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_K, Q6_K, F16])
+def test_batched_many_tokens_non_finite_and_wide_x(g4, ctx, oracle, t):
+    """As for few tokens: infinities and NaN reach their own tokens' outputs as in
+    the sum of the products; the others stay within the bound."""
+    announce("batched many non-finite type %d" % t)
+    m, rows, dim1 = 512, 8192, 1024
+    raw = _no_subnormals(t, synth.weights(68, "mmn%d" % t, t, rows * dim1))
+    X = synth.activations(68, "mmnx", m * dim1).reshape(m, dim1)
+    X[4] *= (10.0 ** np.random.default_rng(68).uniform(-20, 20, dim1)).astype(np.float32)
+    X[1, 5], X[130, 700], X[400, dim1 - 7] = np.inf, np.nan, -np.inf
+    w = upload(g4, ctx, t, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    for i in (0, 1, 4, 129, 130, 131, 400, 511):
+        ex, ab = oracle.matmul_exact(t, raw, X[i], rows, dim1)
+        if i in (1, 130, 400):
+            assert not np.any(np.isfinite(Y[i]))
+            assert np.array_equal(np.isnan(Y[i]), np.isnan(ex)) and np.array_equal(Y[i] > 0, ex > 0)
+        else:
+            assert_dots(Y[i], ex, ab, "token %d" % i)
+    w.free()
+
+
+def test_batched_many_tokens_streams_and_sizes(g4, oracle):
+    """One context's many-token calls on two streams in turn, growing and shrinking,
+    with no synchronisation between them: each result is that of the call alone."""
+    import torch
+    announce("batched many: streams and sizes")
+    rows, dim1 = 8192, 2048
+    raw = synth.weights(69, "mms", Q6_K, rows * dim1)
+    c = g4.Context(0)
+    try:
+        w = upload(g4, c, Q6_K, raw, rows * dim1)
+        X = torch.from_numpy(synth.activations(69, "mmsx", 1300 * dim1).reshape(1300, dim1)).cuda()
+        sizes = [100, 300, 120, 1300, 200, 700]
+        want = []
+        for m in sizes:
+            y = torch.empty((m, rows), device="cuda")
+            w.matmul_batch_dev(X[:m], m, y, rows, dim1)
+            c.sync()
+            want.append(y)
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        torch.cuda.synchronize()
+        for c2 in (c, g4.Context(0)):  # with the workspace there, and from nothing
+            got = [torch.empty_like(y) for y in want]
+            torch.cuda.synchronize()
+            for k, m in enumerate(sizes):
+                c2.set_stream(streams[k % 2].cuda_stream)
+                w2 = w if c2 is c else upload(g4, c2, Q6_K, raw, rows * dim1)
+                w2.matmul_batch_dev(X[:m], m, got[k], rows, dim1)
+            torch.cuda.synchronize()
+            c2.set_stream(None)
+            assert all(torch.equal(a, b) for a, b in zip(want, got))
+            if c2 is not c:
+                c2.close()
+        ex, ab = oracle.matmul_exact(Q6_K, raw, X[1299].cpu().numpy(), rows, dim1)
+        assert_dots(want[3][1299].cpu().numpy(), ex, ab, "token 1299")
+    finally:
+        torch.cuda.synchronize()
+        c.close()
