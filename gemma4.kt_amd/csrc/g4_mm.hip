@@ -33,51 +33,34 @@ constexpr int MM_STAGE_FRAGS = 12;  // a 32-token tile's stage: 4 x 16 columns x
 // bytes hold token l % 32, columns 8 (l / 32) .. + 7.  Tokens past M and columns
 // past dim1 are zeros.  sums[block][token]: the sum over 32 columns.
 //
-// One thread splits a block of one token (128 contiguous bytes); a wave's
-// stores are whole 512-byte runs.
+// A wave splits 16 columns of 32 tokens, eight per lane, and stores three whole
+// operands; a workgroup one stage of a token tile.  Bound by the latency of its
+// loads and stores.  (A whole block of 32 columns per thread left two waves per CU
+// at 512 x 2048: the Q4_K product 65.9-66.3 us, so 64.8-65.1.)
 __global__ __launch_bounds__(256) void k_split(const float *x, int64_t x_stride, int32_t M, int32_t dim1, int32_t stages,
                                                int32_t tiles, unsigned char *planes, float *sums) {
-  const int lane = threadIdx.x & 63, n = lane & 31, b = lane >> 5;
-  const int s = (int)blockIdx.x * 4 + (threadIdx.x >> 6), t = blockIdx.y;
-  if (s >= stages) return;
-  const int tok = t * 32 + n, col = 64 * s + 32 * b;
-  u32x4a4 v[8];
+  __shared__ float half[4][32];
+  const int lane = threadIdx.x & 63, n = lane & 31, k = threadIdx.x >> 6;
+  const int s = blockIdx.x, t = blockIdx.y;
+  const int tok = t * 32 + n, col = 64 * s + 16 * k + 8 * (lane >> 5);
   const bool live = tok < M && col < dim1;
   const u32x4a4 *src = (const u32x4a4 *)(x + (live ? (int64_t)tok * x_stride + col : 0));
+  u32x4a4 u0 = src[0], u1 = src[1];
+  if (!live) u0 = u1 = u32x4a4{0u, 0u, 0u, 0u};
+  const float v[8] = {__uint_as_float(u0.x), __uint_as_float(u0.y), __uint_as_float(u0.z), __uint_as_float(u0.w),
+                      __uint_as_float(u1.x), __uint_as_float(u1.y), __uint_as_float(u1.z), __uint_as_float(u1.w)};
+  // (an infinite x leaves NaN parts: the outputs it reaches are NaN and formed again by k_mm)
+  bf16x8 p[3];
+  split3<false>(v, p[0], p[1], p[2]);
+  unsigned char *dst = planes + (((int64_t)t * stages + s) * MM_STAGE_FRAGS + 3 * k) * MM_FRAG + 16 * lane;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = live ? src[i] : u32x4a4{0u, 0u, 0u, 0u};
-  unsigned char *dst = planes + ((int64_t)t * stages + s) * MM_STAGE_FRAGS * MM_FRAG + 16 * n;
-  float part[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    u32x4 p[3];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      // two values: the truncations to bf16 of x and of x - p1, and the rest, whose
-      // 8 significant bits fit (an infinite x leaves NaN parts: the outputs it
-      // reaches are NaN and formed again by k_mm)
-      uint32_t t1[2], t2[2], t3[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const uint32_t w = v[2 * i + (k >> 1)][2 * (k & 1) + h];
-        t1[h] = w & 0xFFFF0000u;
-        const float r1 = __uint_as_float(w) - __uint_as_float(t1[h]);
-        t2[h] = __float_as_uint(r1) & 0xFFFF0000u;
-        t3[h] = __float_as_uint(r1 - __uint_as_float(t2[h]));
-      }
-      p[0][k] = __builtin_amdgcn_perm(t1[1], t1[0], 0x07060302u);
-      p[1][k] = __builtin_amdgcn_perm(t2[1], t2[0], 0x07060302u);
-      p[2][k] = __builtin_amdgcn_perm(t3[1], t3[0], 0x07060302u);
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) *(u32x4 *)(dst + (3 * (2 * b + (i >> 1)) + q) * MM_FRAG + 512 * (i & 1)) = p[q];
-  }
+  for (int q = 0; q < 3; ++q) *(bf16x8 *)(dst + q * MM_FRAG) = p[q];
   if (sums) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      part[i] = (__uint_as_float(v[i].x) + __uint_as_float(v[i].y)) + (__uint_as_float(v[i].z) + __uint_as_float(v[i].w));
-    sums[(int64_t)(2 * s + b) * (32 * tiles) + tok] =
-        ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    const float sum = pstep<32>(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+    if (lane < 32) half[k][n] = sum;
+    __syncthreads();
+    const int b = lane >> 5;
+    if (k == 0) sums[(int64_t)(2 * s + b) * (32 * tiles) + t * 32 + n] = half[2 * b][n] + half[2 * b + 1][n];
   }
 }
 
@@ -667,7 +650,7 @@ hipError_t launch_mm(int type, const TokArgs &t, void *ws, const DevInfo &dev, h
     p.tiles = (M + 31) / 32;
     p.n_tt = (M + MM_MT - 1) / MM_MT;
     const float *x = t.x + (int64_t)m0 * t.x_stride;
-    hipLaunchKernelGGL(k_split, dim3((unsigned)((p.stages + 3) / 4), (unsigned)p.tiles), dim3(256), 0, s, x, t.x_stride, M,
+    hipLaunchKernelGGL(k_split, dim3((unsigned)p.stages, (unsigned)p.tiles), dim3(256), 0, s, x, t.x_stride, M,
                        t.dim1, p.stages, p.tiles, planes, mins ? sums : (float *)nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
