@@ -27,7 +27,7 @@
 //   Q5_K     18.9 -> 11.6  40.9 -> 15.5  109.1 -> 23.8
 //   Q6_K     24.6 -> 14.6  53.8 -> 20.1  141.8 -> 32.9
 //   BF16     32.5 -> 10.4  90.3 -> 11.8  227.6 -> 16.6  1786 -> 98.5
-//   F16      39.5 -> 19.0 100.7 -> 25.1  245.1 -> 39.0
+//   F16      39.5 -> 16.4 100.7 -> 20.8  245.1 -> 32.0
 // and against 64 bits the error falls from 1.2e-7..3.0e-7 to 1.0e-7..1.4e-7.
 #include "g4_mmfmt.hpp"
 #include "g4_internal.hpp"
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
       float s = v[0];
       const int r = rt * 16 + n, m = 4 * j + wid;
       if (r < a.rows && m < mt) {
-        if (s != s)
+        if (redo<TYPE>(s))
           s = mat_plain_dot<TYPE>(a.W, a.base + (int64_t)r * a.row_stride, a.x + (int64_t)(tok0 + m) * a.x_stride,
                                   sl0 * MAT_COLS, min(a.dim1, (sl0 + nw) * MAT_COLS), a.dim1);
         out[(int64_t)(tok0 + m) * out_stride + r] = s;
@@ -361,7 +361,7 @@ bool mat_ok(int type, const TokArgs &a) {
 //     Q8_0           5.3 / 6.8    5.0 / 6.8   6.4 / 6.8   6.5 / 7.1
 //     Q6_K           6.0 / 9.8    6.2 / 9.8   7.7 / 9.9   8.7 / 9.9
 //     BF16           8.9 / 6.2    7.4 / 6.3   9.7 / 6.4  11.5 / 6.4
-// F16 (8192 x 2048, 3 tokens: 21.4 / 18.4) goes with BF16, Q5_K with the others.
+// F16 (8192 x 2048, 3 tokens: 21.4 / 16.2) goes with BF16, Q5_K with the others.
 int32_t mat_min_tokens(int type, const TokArgs &a) {
   if (type == T_BF16 || type == T_F16) return 3;
   if ((int64_t)a.rows * a.dim1 < (8 << 20)) return 9;

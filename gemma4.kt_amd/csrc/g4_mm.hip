@@ -505,18 +505,18 @@ __global__ __launch_bounds__(MM_THREADS) void k_mm(MmArgs a) {
       const int tok = (t_base + 2 * wm + t) * 32 + 8 * (v >> 2) + 4 * j + (v & 3);
       if (tok < a.M && row < a.rows) {
         out[(int64_t)tok * a.y_stride + row] = sum;
-        bad |= sum != sum;
+        bad |= redo<TYPE>(sum);
       }
     }
   if (bad) {
-    // the lane reads its own outputs back and forms the NaN ones again
+    // the lane reads its own outputs back and forms these again
     const int64_t E = a.base + (int64_t)row * a.row_stride;
 #pragma clang loop unroll(disable)
     for (int q = 0; q < 32; ++q) {
       const int v = q & 15, tok = (t_base + 2 * wm + (q >> 4)) * 32 + 8 * (v >> 2) + 4 * j + (v & 3);
       if (tok >= a.M) continue;
       volatile float *o = out + (int64_t)tok * a.y_stride + row;
-      if (*o != *o)
+      if (redo<TYPE>(*o))
         *o = mm_plain_dot<TYPE>(a.W, E, a.x + (int64_t)tok * a.x_stride, 64 * s0, min(64 * s1, a.dim1), a.dim1);
     }
   }
@@ -589,7 +589,7 @@ hipError_t mm_launch(const MmArgs &a, hipStream_t s) {
 //   Q4_0  2048 x 8192     32.9 / 30.8  57 / 42.0   75 / 67.5  106 / 87.7
 //   Q4_K  8192 x 2048     22.6 / 32.3  37 / 42.9   52 / 59.4   75 / 65.1
 //   Q6_K  8192 x 2048     53.6 / 33.1  93 / 46.1  140 / 65.5  203 / 70.9
-//   F16   8192 x 2048     63.2 / 37.0 116 / 56.8  169 / 96.8  249 / 110
+//   F16   8192 x 2048     63.2 / 37.0 116 / 56.8  169 / 96.8  249 / 110 (f16_parts since faster: 54.2, 111 here)
 //   Q8_0  2048 x 2048     13.1 / 22.7  20 / 24.8   27 / 29.2   38 / 31.4
 static bool mm_faster(int type, const TokArgs &a, const DevInfo &dev) {
   if (a.M <= 64) return false;
@@ -600,7 +600,7 @@ static bool mm_faster(int type, const TokArgs &a, const DevInfo &dev) {
     case T_Q4_0: tile = 1.5; break;
     case T_Q4_K: tile = 1.1; break;
     case T_Q6_K: tile = 3.1; break;
-    default: tile = 3.8; break;
+    default: tile = 3.1; break;
   }
   const int n_sl = (a.dim1 + 127) / 128, splits = (n_sl + 15) / 16, sps = (n_sl + splits - 1) / splits;
   const int wpb = type == T_Q4_K ? 16 : sps <= 4 ? 4 : sps <= 8 ? 8 : 16, n_rt = (a.rows + 15) / 16;

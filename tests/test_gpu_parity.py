@@ -1205,3 +1205,24 @@ def test_batched_many_tokens_streams_and_sizes(g4, oracle):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+@pytest.mark.parametrize("m,rows,dim1", [(5, 20, 512), (512, 8192, 1024)])
+def test_batched_f16_exponent_31(g4, ctx, oracle, m, rows, dim1):
+    """F16 exponent 31 is the finite 2^16 * 1.m in the vector path
+    (F16FloatTensor.kt:59-61): rows with such weights get the one-token call's finite
+    outputs, within the sum of both calls' bounds (1e-5 sum|w x| each)."""
+    announce("batched f16 exponent 31 M=%d" % m)
+    raw = _no_subnormals(F16, synth.weights(64, "mt31.%d" % dim1, F16, rows * dim1)).copy()
+    h = raw.view(np.uint16)
+    h[3 * dim1 + 100], h[7 * dim1 + 5], h[7 * dim1 + 6] = 0x7C00, 0xFE00, 0x7E00
+    X = synth.activations(64, "mt31x%d" % dim1, m * dim1).reshape(m, dim1)
+    w = upload(g4, ctx, F16, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    assert np.all(np.isfinite(Y))
+    for i in (0, 2, m - 1):
+        y = np.empty(rows, np.float32)
+        w.matmul(X[i], y, rows, dim1)
+        bound = 2e-5 * (2.0 ** 17 * np.abs(X[i, [100, 5, 6]]).sum() + np.abs(X[i]).sum())
+        assert np.abs(Y[i, [3, 7]] - y[[3, 7]]).max() <= bound
+    w.free()
