@@ -181,9 +181,10 @@ struct MmStage<T_Q6_K> {
   G4_DEV float offset(int, int) const { return 0.f; }
 };
 
+// (plane 0 the top 8 significant bits, plane 1 the other 3)
 template <>
-struct MmStage<T_BF16> {
-  static constexpr int PLANES = 1, SPB = 0;
+struct MmStage<T_F16> {
+  static constexpr int PLANES = 2, SPB = 0;
   static constexpr bool MIN = false;
   u32x4 q0, q1;
   G4_DEV void arrived() { asm volatile("" : "+v"(q0), "+v"(q1)); }
@@ -192,16 +193,6 @@ struct MmStage<T_BF16> {
     q0 = *(const u32x4 *)p;
     q1 = *(const u32x4 *)(p + 64);
   }
-  G4_DEV bf16x8 lo(int, int, int) const { return __builtin_bit_cast(bf16x8, q0); }
-  G4_DEV bf16x8 hi(int, int, int) const { return __builtin_bit_cast(bf16x8, q1); }
-  G4_DEV float scale(int, int) const { return 1.f; }
-  G4_DEV float offset(int, int) const { return 0.f; }
-};
-
-// (F16: plane 0 the top 8 significant bits, plane 1 the other 3)
-template <>
-struct MmStage<T_F16> : MmStage<T_BF16> {
-  static constexpr int PLANES = 2;
   G4_DEV static bf16x8 plane(const u32x4 &q, int pl) {
     bf16x8 hi, lo;
     f16_parts(q, hi, lo);
@@ -209,6 +200,8 @@ struct MmStage<T_F16> : MmStage<T_BF16> {
   }
   G4_DEV bf16x8 lo(int, int, int pl) const { return plane(q0, pl); }
   G4_DEV bf16x8 hi(int, int, int pl) const { return plane(q1, pl); }
+  G4_DEV float scale(int, int) const { return 1.f; }
+  G4_DEV float offset(int, int) const { return 0.f; }
 };
 
 // ----------------------------------------------------------------- product ---
@@ -599,8 +592,7 @@ static bool mm_faster(int type, const TokArgs &a, const DevInfo &dev) {
     case T_Q8_0: tile = 1.95; break;
     case T_Q4_0: tile = 1.5; break;
     case T_Q4_K: tile = 1.1; break;
-    case T_Q6_K: tile = 3.1; break;
-    default: tile = 3.1; break;
+    default: tile = 3.1; break;  // Q6_K, F16
   }
   const int n_sl = (a.dim1 + 127) / 128, splits = (n_sl + 15) / 16, sps = (n_sl + splits - 1) / splits;
   const int wpb = type == T_Q4_K ? 16 : sps <= 4 ? 4 : sps <= 8 ? 8 : 16, n_rt = (a.rows + 15) / 16;
