@@ -52,12 +52,11 @@ struct g4_ctx {
   int n_outs;
   // Workspace of the tiled many-token product (grow-only), apart from `scratch`:
   // calls that are not being captured use it, so no graph holds its address, and
-  // mm_acquire orders calls on different streams over it.
-  char *mm_ws;
-  size_t mm_bytes;
-  bool mm_used;           // queued work may still use it,
-  hipStream_t mm_stream;  // the last of it on this stream,
-  hipEvent_t mm_event;    // and ended by this event once calls have come on a second stream (else null)
+  // ws_acquire orders calls on different streams over it.
+  char *ws;
+  size_t ws_bytes;
+  enum { WS_IDLE, WS_OWN, WS_CALLER } ws_use;  // queued work may still use it, on own_stream or a caller's stream
+  hipEvent_t ws_event;                         // WS_CALLER: that work is done
 };
 
 struct g4_weight {
@@ -196,64 +195,57 @@ int zero_dev(g4_ctx *ctx, void *p, size_t bytes) {
   return G4_OK;
 }
 
-// The tiled product's workspace of `bytes`, safe to use by work queued on the
-// context's stream from here on; null when the call has to do without: its
-// stream is being captured, the stream of the last use is, or no memory is left.
-// Calls on one stream need no ordering.  The first use on a second stream waits
-// for the last one on the host; from then on every use records an event and a
-// change of stream waits for it on the GPU.
-char *mm_acquire(g4_ctx *ctx, size_t bytes) {
+// The workspace with `bytes`, safe to use by work queued on the context's stream
+// from here on; null when the call has to do without: its stream is being captured,
+// or no memory is left.  A change of stream waits on the GPU: for an event recorded
+// behind the last use if that was on a caller's stream (which may be gone by now,
+// its handle another stream's), else for one recorded on own_stream here.
+char *ws_acquire(g4_ctx *ctx, size_t bytes) {
   if (ctx->capturing) return nullptr;
-  const bool grow = bytes > ctx->mm_bytes, moved = ctx->mm_used && ctx->mm_stream != ctx->stream;
-  if (!grow && !moved) return ctx->mm_ws;
-  if (!grow && ctx->mm_event) {
-    if (hipStreamWaitEvent(ctx->stream, ctx->mm_event, 0) == hipSuccess) return ctx->mm_ws;
+  // another thread's capture is not disturbed by the allocation and the waits
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  // another thread's capture is not disturbed by the allocation and the waits
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
   bool ok = true;
-  if (ctx->mm_used) {
-    if (ctx->mm_event) {
-      ok = hipEventSynchronize(ctx->mm_event) == hipSuccess;
-    } else {
-      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing(ctx->mm_stream, &st) != hipSuccess)
-        ok = hipDeviceSynchronize() == hipSuccess;  // the stream is gone
-      else
-        ok = st == hipStreamCaptureStatusNone && hipStreamSynchronize(ctx->mm_stream) == hipSuccess;
-    }
-    if (ok) ctx->mm_used = false;
-  }
-  if (ok && moved && !ctx->mm_event && hipEventCreateWithFlags(&ctx->mm_event, hipEventDisableTiming) != hipSuccess) {
-    ctx->mm_event = nullptr;
+  if (!ctx->ws_event && hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming) != hipSuccess) {
+    ctx->ws_event = nullptr;
     ok = false;
   }
-  if (ok && grow) {
-    if (ctx->mm_ws) (void)hipFree(ctx->mm_ws);
-    ctx->mm_ws = nullptr;
-    ctx->mm_bytes = 0;
-    const size_t want = std::max(bytes, size_t(64) << 20);
-    void *p = nullptr;
-    if (hipMalloc(&p, want) == hipSuccess) {
-      ctx->mm_ws = (char *)p;
-      ctx->mm_bytes = want;
-    } else {
-      ok = false;
+  if (ok && bytes > ctx->ws_bytes) {
+    if (ctx->ws_use == g4_ctx::WS_OWN)
+      ok = hipStreamSynchronize(ctx->own_stream) == hipSuccess;
+    else if (ctx->ws_use == g4_ctx::WS_CALLER)
+      ok = hipEventSynchronize(ctx->ws_event) == hipSuccess;
+    if (ok) {
+      ctx->ws_use = g4_ctx::WS_IDLE;
+      if (ctx->ws) (void)hipFree(ctx->ws);
+      ctx->ws = nullptr;
+      ctx->ws_bytes = 0;
+      const size_t want = std::max(bytes, size_t(64) << 20);
+      void *p = nullptr;
+      ok = hipMalloc(&p, want) == hipSuccess;
+      if (ok) {
+        ctx->ws = (char *)p;
+        ctx->ws_bytes = want;
+      }
     }
+  } else if (ok && ctx->ws_use == g4_ctx::WS_CALLER) {
+    ok = hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0) == hipSuccess;
+  } else if (ok && ctx->ws_use == g4_ctx::WS_OWN && ctx->stream != ctx->own_stream) {
+    ok = hipEventRecord(ctx->ws_event, ctx->own_stream) == hipSuccess &&
+         hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0) == hipSuccess;
   }
   (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (!ok) (void)hipGetLastError();  // the caller takes another route
-  return ok ? ctx->mm_ws : nullptr;
+  if (!ok) (void)hipGetLastError();  // the caller takes another route, whose launches read the last error
+  return ok ? ctx->ws : nullptr;
 }
 
 // The workspace's use is queued on the context's stream.
-int mm_release(g4_ctx *ctx) {
-  ctx->mm_used = true;
-  ctx->mm_stream = ctx->stream;
-  if (ctx->mm_event) G4_HIP(hipEventRecord(ctx->mm_event, ctx->stream), "hipEventRecord");
+int ws_release(g4_ctx *ctx) {
+  ctx->ws_use = ctx->stream == ctx->own_stream ? g4_ctx::WS_OWN : g4_ctx::WS_CALLER;
+  if (ctx->ws_use == g4_ctx::WS_CALLER) G4_HIP(hipEventRecord(ctx->ws_event, ctx->stream), "hipEventRecord");
   return G4_OK;
 }
 
@@ -460,7 +452,7 @@ BatchRoute batch_route(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, 
   if (M < 3 || dim0 == 0 || dim1 == 0) return {BatchRoute::ROWS, 0, nullptr};
   const g4::TokArgs t = tok_args(w, off, nullptr, M, nullptr, dim0, dim1);
   if (g4::mm_ok(w->type, t, ctx->dev))
-    if (char *ws = mm_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))) return {BatchRoute::MM, 0, ws};
+    if (char *ws = ws_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))) return {BatchRoute::MM, 0, ws};
   // Two tokens stay on the row engine: measured on 8192 x 2048 Q4_K, 6.5 us against
   // 8.9 us for the matrix cores; from three on the matrix cores are as fast or
   // faster (9.1 / 9.3 us at M = 3, 9.6 / 14.4 at M = 8).  For the other formats
@@ -493,7 +485,7 @@ int batch_dev(g4_ctx *ctx, const g4_weight *w, int64_t off, const float *d_X, in
   }
   if (r.kind == BatchRoute::MM) {
     const hipError_t e = g4::launch_mm(w->type, tok_args(w, off, d_X, M, d_Y, dim0, dim1), r.ws, ctx->dev, ctx->stream);
-    G4_TRY(mm_release(ctx));
+    G4_TRY(ws_release(ctx));
     return launch_status(e, "matmul_batch");
   }
   if (r.kind != BatchRoute::ROWS) {
@@ -931,11 +923,11 @@ int g4_close(g4_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   (void)hipStreamSynchronize(ctx->own_stream);
-  if (ctx->mm_event) {
-    (void)hipEventSynchronize(ctx->mm_event);
-    (void)hipEventDestroy(ctx->mm_event);
+  if (ctx->ws_event) {
+    if (ctx->ws_use == g4_ctx::WS_CALLER) (void)hipEventSynchronize(ctx->ws_event);
+    (void)hipEventDestroy(ctx->ws_event);
   }
-  if (ctx->mm_ws) (void)hipFree(ctx->mm_ws);
+  if (ctx->ws) (void)hipFree(ctx->ws);
   if (ctx->scratch) (void)hipFree(ctx->scratch);
   for (int i = 0; i < ctx->n_retired; ++i) (void)hipFree(ctx->retired[i]);
   if (ctx->am_val) (void)hipFree(ctx->am_val);

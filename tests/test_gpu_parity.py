@@ -7,6 +7,8 @@ Bars (written into each check):
     the same bound, tests/test_oracle_pins.py);
   * argmax indices, routing ids and routing weights: exact.
 """
+import os
+
 import numpy as np
 import pytest
 
@@ -1202,6 +1204,37 @@ def test_batched_many_tokens_streams_and_sizes(g4, oracle):
                 c2.close()
         ex, ab = oracle.matmul_exact(Q6_K, raw, X[1299].cpu().numpy(), rows, dim1)
         assert_dots(want[3][1299].cpu().numpy(), ex, ab, "token 1299")
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
+def test_batched_many_tokens_after_their_stream_is_gone(g4):
+    """The stream of the last many-token call is destroyed, its work done, before the
+    next one: same bits."""
+    import ctypes
+    import torch
+    announce("batched many: stream gone")
+    hip = ctypes.CDLL(os.path.join(torch.__path__[0], "lib", "libamdhip64.so"))  # (the one the library binds to)
+    m, rows, dim1 = 300, 8192, 2048
+    c = g4.Context(0)
+    try:
+        w = upload(g4, c, Q6_K, synth.weights(69, "mms", Q6_K, rows * dim1), rows * dim1)
+        X = torch.from_numpy(synth.activations(69, "mmsx", m * dim1).reshape(m, dim1)).cuda()
+        torch.cuda.synchronize()
+        got = []
+        for _ in range(3):
+            s = ctypes.c_void_p()
+            assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+            c.set_stream(s.value)
+            y = torch.zeros((m, rows), device="cuda")
+            torch.cuda.synchronize()
+            w.matmul_batch_dev(X, m, y, rows, dim1)
+            assert hip.hipStreamSynchronize(s) == 0 and hip.hipStreamDestroy(s) == 0
+            got.append(y)
+        c.set_stream(None)
+        assert bool(got[0].any()) and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+        w.free()
     finally:
         torch.cuda.synchronize()
         c.close()

@@ -1,0 +1,204 @@
+"""The library's host code on the CPU: its sources compiled for the host only and
+linked to a stand-in for the HIP runtime (tests/host/hip_stub.cpp) that logs each
+launch, event and wait with its stream.  Shown here is what no GPU run shows
+reliably: which kernels a call takes, how calls on several streams are ordered
+over a shared workspace, and what a call does when memory runs out or a stream is
+gone."""
+import ctypes
+import os
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+import build as pkg_build
+import g4hip
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+Q8_0, Q4_0, Q4_K, Q5_K, Q6_K, F16, BF16 = 8, 2, 12, 13, 14, 1, 30
+KERNELS = ["k_split", "k_mm", "k_tok_q4k", "k_tok_reduce", "k_mat", "k_rows", "k_wide"]
+
+
+def _run(cmd):
+    p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert p.returncode == 0, p.stdout
+    return p.stdout
+
+
+@pytest.fixture(scope="module")
+def hip(tmp_path_factory):
+    d = str(tmp_path_factory.mktemp("host"))
+    host = [pkg_build.HIPCC, "-O1", "-std=c++17", "-fPIC", "-w", "-c"]
+    jobs = [host + [os.path.join(HERE, "host", "hip_stub.cpp"), "-o", os.path.join(d, "stub.o")]]
+    for src in pkg_build.SOURCES:
+        jobs.append(host + ["--offload-host-only", "--offload-arch=" + pkg_build.ARCH, "-I",
+                            os.path.join(pkg_build.ROOT, "include"), os.path.join(pkg_build.CSRC, src), "-o",
+                            os.path.join(d, src + ".o")])
+    with ThreadPoolExecutor(len(jobs)) as ex:
+        list(ex.map(_run, jobs))
+    objs = [j[-1] for j in jobs]
+    # the device code that the host objects refer to is not there
+    fat = {w for l in _run(["nm", "-u"] + objs).splitlines() for w in l.split() if w.startswith("__hip_fatbin")}
+    so = os.path.join(d, "libg4host.so")
+    _run(["g++", "-shared", "-Wl,-Bsymbolic"] + ["-Wl,--defsym=%s=0" % f for f in sorted(fat)] + ["-o", so] + objs)
+    L = ctypes.CDLL(so)
+    for name, args in g4hip.SIGNATURES.items():
+        getattr(L, name).argtypes = args
+    L.g4_last_error.restype = L.stub_log.restype = ctypes.c_char_p
+    L.stub_free_bytes.argtypes = [ctypes.c_size_t]
+    L.stub_capture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    L.stub_stream_id.argtypes = L.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    yield L
+    L.stub_free_bytes(ctypes.c_size_t(-1).value)
+
+
+class Program:
+    """One context and a weight of every size asked for; its calls as a program makes them."""
+
+    def __init__(self, hip):
+        self.hip, self.weights = hip, {}
+        hip.stub_free_bytes(ctypes.c_size_t(-1).value)
+        hip.hipGetLastError()
+        self.ctx = ctypes.c_void_p()
+        assert hip.g4_open(0, ctypes.byref(self.ctx)) == 0
+        hip.stub_clear()
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        self.hip.stub_free_bytes(ctypes.c_size_t(-1).value)
+        for w in self.weights.values():
+            self.hip.g4_weight_free(w)
+        assert self.hip.g4_close(self.ctx) == 0
+
+    def stream(self):
+        s = ctypes.c_void_p()
+        assert self.hip.hipStreamCreateWithFlags(ctypes.byref(s), 0) == 0
+        return s
+
+    def use(self, stream):
+        assert self.hip.g4_ctx_set_stream(self.ctx, stream) == 0
+
+    def batch(self, t, m, rows, cols):
+        """matmul_batch_dev; the names of the kernels it launched."""
+        key = (t, rows * cols)
+        if key not in self.weights:
+            n = (ctypes.c_int64 * 1)()
+            assert self.hip.g4_byte_size(t, rows * cols, n) == 0
+            w = (ctypes.c_void_p * 1)()
+            assert self.hip.g4_upload(self.ctx, t, ctypes.create_string_buffer(n[0]), n[0], rows * cols, w) == 0
+            w = w[0]
+            self.weights[key] = w
+        before = len(self.log())
+        rc = self.hip.g4_matmul_batch_dev(self.ctx, self.weights[key], 0, 4096, m, 8192, rows, cols)
+        assert rc == 0, self.hip.g4_last_error()
+        return [self.kernel(l[1]) for l in self.log()[before:] if l[0] == "launch"]
+
+    def log(self):
+        return [l.split() for l in self.hip.stub_log().decode().splitlines()]
+
+    @staticmethod
+    def kernel(name):
+        return next((k for k in KERNELS if "%d%s" % (len(k), k) in name), name)
+
+    def assert_ordered(self):
+        """Every launch that uses a workspace comes after the previous one that used
+        the same memory, in stream order or over events and waits of the host."""
+        streams, events, host, used, planes = {}, {}, {}, {}, {}
+
+        def merge(a, b):
+            for k, v in b.items():
+                a[k] = max(a.get(k, 0), v)
+
+        for l in self.log():
+            if l[0] == "launch":
+                k, s = self.kernel(l[1]), l[2]
+                c = streams.setdefault(s, {})
+                merge(c, host)
+                ws = [l[3]] if len(l) > 3 else []
+                if k == "k_split":
+                    planes[s] = l[3]
+                elif k in ("k_mm", "k_tok_reduce") and s in planes:
+                    ws.append(planes[s])  # of its k_split
+                for w in ws:
+                    for other, n in used.get(w, {}).items():
+                        assert c.get(other, 0) >= n, "unordered use of the workspace: %s" % l
+                c[s] = c.get(s, 0) + 1
+                for w in ws:
+                    used[w] = {s: c[s]}
+            elif l[0] == "record":
+                events[l[1]] = dict(streams.setdefault(l[2], {}))
+            elif l[0] == "wait":
+                merge(streams.setdefault(l[1], {}), events.get(l[2], {}))
+            elif l[0] == "sync":
+                merge(host, streams.get(l[1], {}))
+            elif l[0] == "sync_event":
+                merge(host, events.get(l[1], {}))
+            elif l[0] in ("sync_device", "free"):  # (hipFree waits for the device)
+                for c in streams.values():
+                    merge(host, c)
+                if l[0] == "free":
+                    used.pop(l[1], None)
+
+
+# many-token calls that take the tiled product (its planes and split sums are in a
+# workspace of the context)
+MANY = [(Q6_K, 512, 8192, 2048), (Q4_0, 201, 2048, 8192), (Q4_K, 512, 8192, 2048)]
+
+
+@pytest.mark.parametrize("t,m,rows,cols", MANY)
+def test_many_token_calls_on_several_streams_are_ordered(hip, t, m, rows, cols):
+    with Program(hip) as p:
+        streams = [None, p.stream(), p.stream()]
+        for k in (0, 0, 1, 2, 2, 1, 0, 1):
+            p.use(streams[k])
+            assert "k_mm" in p.batch(t, m, rows, cols)
+        p.assert_ordered()
+
+
+@pytest.mark.parametrize("same_handle", [False, True])
+def test_many_token_calls_after_their_stream_is_gone(hip, same_handle):
+    """The stream of the last call has been destroyed: the next call runs all its
+    kernels and succeeds, also where the runtime gives the same handle out again
+    while that call's work may not be done."""
+    with Program(hip) as p:
+        a = p.stream()
+        b = None if same_handle else p.stream()
+        p.use(a)
+        p.batch(*MANY[0])
+        hip.hipStreamDestroy(a)
+        b = b or p.stream()
+        assert (a.value == b.value) == same_handle
+        p.use(b)
+        assert p.batch(*MANY[0]) == ["k_split", "k_mm"]
+        p.use(None)
+        assert p.batch(*MANY[0]) == ["k_split", "k_mm"]
+        assert hip.stub_last_error() == 0
+        p.assert_ordered()
+
+
+def test_many_token_call_without_memory_for_its_workspace(hip):
+    with Program(hip) as p:
+        p.batch(Q6_K, 2, 8192, 2048)  # (uploads)
+        p.hip.stub_free_bytes(1 << 20)
+        assert p.batch(Q6_K, 512, 8192, 2048) == ["k_mat"]
+        assert p.hip.stub_last_error() == 0
+
+
+def test_many_token_call_beside_another_streams_capture(hip):
+    """A capture on another stream, the one of the last call among them, does not
+    change which kernels a call runs."""
+    with Program(hip) as p:
+        a = p.stream()
+        p.use(a)
+        p.batch(Q6_K, 2, 16384, 2048)  # (uploads)
+        p.batch(*MANY[0])
+        p.hip.stub_capture(a, 1)
+        p.use(None)
+        assert p.batch(*MANY[0]) == ["k_split", "k_mm"]
+        assert p.batch(Q6_K, 1024, 16384, 2048) == ["k_split", "k_mm"]
+        p.hip.stub_capture(a, 0)
+        p.use(a)
+        p.batch(*MANY[0])
+        p.assert_ordered()
