@@ -448,17 +448,15 @@ struct BatchRoute {
 // Several tokens of one matrix: the matrix-core kernels unpack each weight once
 // for 16 of them (Q4_K: g4_tok.hip, the other formats: g4_mat.hip), or for 128
 // (g4_mm.hip) where there is a workspace; the row engine runs one segment per token.
-BatchRoute batch_route(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1) {
-  if (M < 3 || dim0 == 0 || dim1 == 0) return {BatchRoute::ROWS, 0, nullptr};
-  const g4::TokArgs t = tok_args(w, off, nullptr, M, nullptr, dim0, dim1);
-  if (g4::mm_ok(w->type, t, ctx->dev))
-    if (char *ws = ws_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))) return {BatchRoute::MM, 0, ws};
+// This is the route without the workspace.
+BatchRoute scratch_route(const g4_ctx *ctx, const g4_weight *w, const g4::TokArgs &t) {
   // Two tokens stay on the row engine: measured on 8192 x 2048 Q4_K, 6.5 us against
   // 8.9 us for the matrix cores; from three on the matrix cores are as fast or
   // faster (9.1 / 9.3 us at M = 3, 9.6 / 14.4 at M = 8).  For the other formats
   // mat_min_tokens draws the line.
+  if (t.M < 3 || t.rows == 0 || t.dim1 == 0) return {BatchRoute::ROWS, 0, nullptr};
   if (g4::tok_ok(w->type, t)) return {BatchRoute::TOK, g4::tok_scratch_floats(t, ctx->dev), nullptr};
-  if (M >= g4::mat_min_tokens(w->type, t) && g4::mat_ok(w->type, t))
+  if (t.M >= g4::mat_min_tokens(w->type, t) && g4::mat_ok(w->type, t))
     return {BatchRoute::MAT, g4::mat_scratch_floats(t, ctx->dev), nullptr};
   return {BatchRoute::ROWS, 0, nullptr};
 }
@@ -469,8 +467,18 @@ BatchRoute batch_route(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, 
 // memory left).
 int batch_prepare(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1, size_t before,
                   BatchRoute *r) {
-  *r = batch_route(ctx, w, off, M, dim0, dim1);
-  const int rc = ensure_scratch(ctx, before + sizeof(float) * (size_t)r->part);
+  const g4::TokArgs t = tok_args(w, off, nullptr, M, nullptr, dim0, dim1);
+  *r = scratch_route(ctx, w, t);
+  const size_t bytes = before + sizeof(float) * (size_t)r->part;
+  if (g4::mm_ok(w->type, t, ctx->dev))
+    if (char *ws = ws_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))) {
+      // The same call takes the other route when its stream is being captured: an
+      // eager run of it leaves the scratch for that (if there is the memory).
+      if (ensure_scratch(ctx, bytes) != G4_OK) (void)hipGetLastError();
+      *r = {BatchRoute::MM, 0, ws};
+      return ensure_scratch(ctx, before);
+    }
+  const int rc = ensure_scratch(ctx, bytes);
   if (rc == G4_OK || r->kind != BatchRoute::MAT || r->part == 0) return rc;
   *r = {BatchRoute::ROWS, 0, nullptr};
   return ensure_scratch(ctx, before);

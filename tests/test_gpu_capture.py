@@ -299,3 +299,40 @@ def test_batched_wide_rows_captured(g4, reserve):
     finally:
         torch.cuda.synchronize()
         c.close()
+
+
+@pytest.mark.parametrize("t", [12, 8])
+def test_batched_prompt_captured_after_an_eager_run(g4, t):
+    """A prompt on wide rows, run once eagerly (the tiled product with its workspace)
+    and then captured with nothing reserved: the eager run left the scratch that the
+    captured kernels need."""
+    announce("capture: prompt after an eager run, type %d" % t)
+    m, rows, cols = 512, 2048, 8192
+    raw = synth.weights(47, "bp%d" % t, t, rows * cols)
+    X = torch.from_numpy(synth.activations(47, "bpx", m * cols).reshape(m, cols)).cuda()
+    Y = torch.empty((m, rows), device="cuda")
+    c = g4.Context(0)
+    stream = torch.cuda.Stream()
+    try:
+        w = g4.FloatTensorFactory.create(c, t, raw, rows * cols)
+        w.matmul_batch_dev(X, m, Y, rows, cols)
+        c.sync()
+        eager, before = Y.clone(), c.scratch_bytes()
+        g = _capture(c, stream, lambda: w.matmul_batch_dev(X, m, Y, rows, cols))
+        assert c.scratch_bytes() == before
+        # fp32 sums in another order: both within 1e-5 sum|w x| of exact (test_gpu_parity)
+        bound = 2e-5 * float(abs(X).sum(1).max()) * float(abs(torch.from_numpy(w.dequant(0, rows * cols))).max())
+        first = None
+        for _ in range(3):
+            Y.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            first = Y.clone() if first is None else first
+            assert torch.equal(Y, first) and float((Y - eager).abs().max()) <= bound
+            w.matmul_batch_dev(X, m, Y, rows, cols)  # eager work between the replays
+            c.sync()
+            assert torch.equal(Y, eager)
+        w.free()
+    finally:
+        torch.cuda.synchronize()
+        c.close()

@@ -202,3 +202,20 @@ def test_many_token_call_beside_another_streams_capture(hip):
         p.use(a)
         p.batch(*MANY[0])
         p.assert_ordered()
+
+
+@pytest.mark.parametrize("t,m,rows,cols", [(Q4_K, 512, 2048, 8192), (Q4_K, 512, 4096, 4096), (Q4_K, 201, 2560, 10240),
+                                           (Q8_0, 512, 2048, 8192), (Q4_0, 201, 2048, 8192), (Q6_K, 300, 2048, 8192)])
+def test_an_eager_call_leaves_the_scratch_for_its_capture(hip, t, m, rows, cols):
+    """include/g4hip.h: run the largest shapes once eagerly before capturing.  The
+    eager calls here take the tiled product, the captured ones the 16-token tiles
+    with their split sums in the scratch."""
+    with Program(hip) as p:
+        s = p.stream()
+        p.use(s)
+        assert "k_mm" in p.batch(t, m, rows, cols)
+        hip.stub_clear()
+        hip.stub_capture(s, 1)
+        assert p.batch(t, m, rows, cols) == ["k_tok_q4k" if t == Q4_K else "k_mat", "k_tok_reduce"]
+        assert not [l for l in p.log() if l[0] == "malloc"]
+        hip.stub_capture(s, 0)
