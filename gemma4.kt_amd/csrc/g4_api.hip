@@ -50,7 +50,7 @@ struct g4_ctx {
   size_t pin_used;
   G4PendingOut outs[8];
   int n_outs;
-  // Workspace of the tiled many-token product (grow-only), apart from `scratch`:
+  // Workspace of the several-token products (grow-only), apart from `scratch`:
   // calls that are not being captured use it, so no graph holds its address, and
   // ws_acquire orders calls on different streams over it.
   char *ws;
@@ -442,7 +442,7 @@ g4::TokArgs tok_args(const g4_weight *w, int64_t off, const float *d_X, int32_t 
 struct BatchRoute {
   enum Kind { ROWS, TOK, MAT, MM } kind;
   int64_t part;
-  char *ws;  // MM: the tiled product's workspace
+  char *ws;  // the workspace, where it is used: MM, and MAT's partial sums
 };
 
 // Several tokens of one matrix: the matrix-core kernels unpack each weight once
@@ -462,25 +462,29 @@ BatchRoute scratch_route(const g4_ctx *ctx, const g4_weight *w, const g4::TokArg
 }
 
 // The route of a call that needs `before` bytes of scratch besides, with that
-// scratch there.  A call of the formats the row engine takes without scratch
-// falls back to it where no scratch can be had (none reserved under a capture, no
-// memory left).
+// scratch there.  The types other than Q4_K leave the scratch to captured calls: it
+// is the same memory for every stream and graph, and one segment of the row engine
+// per token, which they can do with, needs none.
 int batch_prepare(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32_t dim0, int32_t dim1, size_t before,
                   BatchRoute *r) {
   const g4::TokArgs t = tok_args(w, off, nullptr, M, nullptr, dim0, dim1);
   *r = scratch_route(ctx, w, t);
   const size_t bytes = before + sizeof(float) * (size_t)r->part;
-  if (g4::mm_ok(w->type, t, ctx->dev))
-    if (char *ws = ws_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))) {
-      // The same call takes the other route when its stream is being captured: an
-      // eager run of it leaves the scratch for that (if there is the memory).
-      if (ensure_scratch(ctx, bytes) != G4_OK) (void)hipGetLastError();
-      *r = {BatchRoute::MM, 0, ws};
-      return ensure_scratch(ctx, before);
-    }
-  const int rc = ensure_scratch(ctx, bytes);
-  if (rc == G4_OK || r->kind != BatchRoute::MAT || r->part == 0) return rc;
-  *r = {BatchRoute::ROWS, 0, nullptr};
+  if (ctx->capturing) {
+    if (r->kind == BatchRoute::MAT && bytes > ctx->scratch_bytes) *r = {BatchRoute::ROWS, 0, nullptr};
+    return ensure_scratch(ctx, before + sizeof(float) * (size_t)r->part);
+  }
+  char *ws = nullptr;
+  if (g4::mm_ok(w->type, t, ctx->dev) && (ws = ws_acquire(ctx, g4::mm_ws_bytes(w->type, t, ctx->dev))))
+    r->kind = BatchRoute::MM;
+  else if (r->kind == BatchRoute::MAT && r->part > 0 && !(ws = ws_acquire(ctx, sizeof(float) * (size_t)r->part)))
+    *r = {BatchRoute::ROWS, 0, nullptr};
+  if (!ws) return ensure_scratch(ctx, before + sizeof(float) * (size_t)r->part);
+  // Captured, the same call needs the scratch: an eager run of it leaves that (if
+  // there is the memory).
+  if (ensure_scratch(ctx, bytes) != G4_OK) (void)hipGetLastError();
+  r->part = 0;
+  r->ws = ws;
   return ensure_scratch(ctx, before);
 }
 
@@ -491,17 +495,14 @@ int batch_dev(g4_ctx *ctx, const g4_weight *w, int64_t off, const float *d_X, in
     G4_TRY(zero_dev(ctx, d_Y, sizeof(float) * (size_t)dim0 * M));
     return G4_OK;
   }
-  if (r.kind == BatchRoute::MM) {
-    const hipError_t e = g4::launch_mm(w->type, tok_args(w, off, d_X, M, d_Y, dim0, dim1), r.ws, ctx->dev, ctx->stream);
-    G4_TRY(ws_release(ctx));
-    return launch_status(e, "matmul_batch");
-  }
   if (r.kind != BatchRoute::ROWS) {
     g4::TokArgs t = tok_args(w, off, d_X, M, d_Y, dim0, dim1);
-    t.part = r.part > 0 ? d_part : nullptr;
-    return launch_status(r.kind == BatchRoute::TOK ? g4::launch_tok(w->type, t, ctx->dev, ctx->stream)
-                                                   : g4::launch_mat(w->type, t, ctx->dev, ctx->stream),
-                         "matmul_batch");
+    t.part = r.ws ? (float *)r.ws : r.part > 0 ? d_part : nullptr;
+    const hipError_t e = r.kind == BatchRoute::MM    ? g4::launch_mm(w->type, t, r.ws, ctx->dev, ctx->stream)
+                         : r.kind == BatchRoute::TOK ? g4::launch_tok(w->type, t, ctx->dev, ctx->stream)
+                                                     : g4::launch_mat(w->type, t, ctx->dev, ctx->stream);
+    if (r.ws) G4_TRY(ws_release(ctx));
+    return launch_status(e, "matmul_batch");
   }
   g4::RowsArgs a = plain_rows(w, off, d_X, d_Y, dim0, dim1);
   a.x_stride = dim1;

@@ -368,26 +368,41 @@ int32_t mat_min_tokens(int type, const TokArgs &a) {
   return a.dim1 > 16 * MAT_COLS ? 6 : 4;
 }
 
-int64_t mat_scratch_floats(const TokArgs &a, const DevInfo &dev) {
-  const MatShape sh = mat_shape(a, dev);
-  return sh.splits > 1 ? (int64_t)sh.splits * a.M * a.rows : 0;
+// Tokens per pass: as many as MAT_PART_FLOATS holds the column splits' sums of.
+constexpr int64_t MAT_PART_FLOATS = int64_t(16) << 20;
+static int32_t mat_pass(const TokArgs &a, const MatShape &sh) {
+  if (sh.splits == 1) return a.M;
+  return (int32_t)std::min<int64_t>(a.M, std::max<int64_t>(16, MAT_PART_FLOATS / ((int64_t)sh.splits * a.rows) / 16 * 16));
 }
 
-hipError_t launch_mat(int type, const TokArgs &a, const DevInfo &dev, hipStream_t s) {
-  if (!mat_ok(type, a)) return hipErrorInvalidValue;
+int64_t mat_scratch_floats(const TokArgs &a, const DevInfo &dev) {
   const MatShape sh = mat_shape(a, dev);
-  if (sh.splits > 1 && !a.part) return hipErrorInvalidValue;
-  hipError_t e;
-  switch (type) {
-    case T_Q8_0: e = launch_mat_t<T_Q8_0>(a, sh, s); break;
-    case T_Q4_0: e = launch_mat_t<T_Q4_0>(a, sh, s); break;
-    case T_Q5_K: e = launch_mat_t<T_Q5_K>(a, sh, s); break;
-    case T_Q6_K: e = launch_mat_t<T_Q6_K>(a, sh, s); break;
-    case T_BF16: e = launch_mat_t<T_BF16>(a, sh, s); break;
-    default: e = launch_mat_t<T_F16>(a, sh, s); break;
+  return sh.splits > 1 ? (int64_t)sh.splits * mat_pass(a, sh) * a.rows : 0;
+}
+
+hipError_t launch_mat(int type, const TokArgs &t, const DevInfo &dev, hipStream_t s) {
+  if (!mat_ok(type, t)) return hipErrorInvalidValue;
+  const int32_t pass = mat_pass(t, mat_shape(t, dev));
+  TokArgs a = t;
+  for (int32_t m0 = 0; m0 < t.M; m0 += pass) {
+    a.M = std::min(pass, t.M - m0);
+    a.x = t.x + (int64_t)m0 * t.x_stride;
+    a.y = t.y + (int64_t)m0 * t.y_stride;
+    const MatShape sh = mat_shape(a, dev);
+    if (sh.splits > 1 && !a.part) return hipErrorInvalidValue;
+    hipError_t e;
+    switch (type) {
+      case T_Q8_0: e = launch_mat_t<T_Q8_0>(a, sh, s); break;
+      case T_Q4_0: e = launch_mat_t<T_Q4_0>(a, sh, s); break;
+      case T_Q5_K: e = launch_mat_t<T_Q5_K>(a, sh, s); break;
+      case T_Q6_K: e = launch_mat_t<T_Q6_K>(a, sh, s); break;
+      case T_BF16: e = launch_mat_t<T_BF16>(a, sh, s); break;
+      default: e = launch_mat_t<T_F16>(a, sh, s); break;
+    }
+    if (e == hipSuccess && sh.splits > 1) e = launch_tok_reduce(a.part, sh.splits, a.M, a.rows, a.y, a.y_stride, s);
+    if (e != hipSuccess) return e;
   }
-  if (e != hipSuccess || sh.splits == 1) return e;
-  return launch_tok_reduce(a.part, sh.splits, a.M, a.rows, a.y, a.y_stride, s);
+  return hipSuccess;
 }
 
 }  // namespace g4

@@ -17,6 +17,8 @@
 #include <map>
 #include <string>
 
+#include "../../gemma4.kt_amd/csrc/g4_internal.hpp"
+
 namespace {
 
 hipError_t last = hipSuccess;
@@ -180,9 +182,11 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
   Stream *p = at(s);
   if (!p) return fail(hipErrorContextIsDestroyed);
   const std::string &k = kernels[f];
-  // the workspace a kernel writes (k_split: its seventh argument) or reads
-  // (k_tok_reduce: its first)
+  // the workspace a kernel writes (k_split: its seventh argument; the 16-token tiles:
+  // the partial sums) or reads (k_tok_reduce: its first)
   void *ws = nullptr;
+  if (k.find("k_mat") != std::string::npos || k.find("k_tok_q4k") != std::string::npos)
+    ws = ((const g4::TokArgs *)args[0])->part;
   if (k.find("k_split") != std::string::npos) memcpy(&ws, args[6], sizeof(ws));
   if (k.find("k_tok_reduce") != std::string::npos) memcpy(&ws, args[0], sizeof(ws));
   if (ws)

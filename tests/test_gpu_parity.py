@@ -1021,6 +1021,58 @@ def test_batched_matrix_core_few_tokens(g4, ctx, oracle, t, m, rows, dim1):
     _batched_case(g4, ctx, oracle, t, m, rows, dim1, 0)
 
 
+def test_batched_wide_rows_in_passes(g4, ctx, oracle):
+    """Column splits of more tokens than their sums are held for at a time (three
+    splits of 8192 rows: 672 tokens)."""
+    announce("batched wide rows in passes")
+    m, rows, dim1 = 700, 8192, 4160
+    raw = synth.weights(61, "mtp", BF16, rows * dim1)
+    X = synth.activations(61, "mtpx", m * dim1).reshape(m, dim1)
+    w = upload(g4, ctx, BF16, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    for i in (0, 671, 672, 699):
+        ex, ab = oracle.matmul_exact(BF16, raw, X[i], rows, dim1)
+        assert_dots(Y[i], ex, ab, "token %d" % i)
+    # every token: the same sums in the same order
+    assert same_bits(Y[:350], w.matmul_batch(X[:350], rows, dim1))
+    assert same_bits(Y[350:], w.matmul_batch(X[350:], rows, dim1))
+    w.free()
+
+
+@pytest.mark.parametrize("t", [Q8_0, BF16])
+def test_batched_wide_rows_streams(g4, oracle, t):
+    """Calls with column splits on two streams in turn, with no synchronisation
+    between them: each result is that of the call alone."""
+    import torch
+    announce("batched wide rows: streams, type %d" % t)
+    rows, dim1 = 2048, 8192
+    raw = synth.weights(61, "mts%d" % t, t, rows * dim1)
+    X = torch.from_numpy(synth.activations(61, "mtsx", 64 * dim1).reshape(64, dim1)).cuda()
+    sizes = [12, 64, 9, 40, 17, 33] * 3
+    c = g4.Context(0)
+    try:
+        w = upload(g4, c, t, raw, rows * dim1)
+        want, got = [], [torch.empty((m, rows), device="cuda") for m in sizes]
+        for m in sizes:
+            want.append(torch.empty((m, rows), device="cuda"))
+            w.matmul_batch_dev(X[:m], m, want[-1], rows, dim1)
+            c.sync()
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        torch.cuda.synchronize()
+        for k, m in enumerate(sizes):
+            c.set_stream(streams[k % 2].cuda_stream)
+            w.matmul_batch_dev(X[:m], m, got[k], rows, dim1)
+        torch.cuda.synchronize()
+        c.set_stream(None)
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
+        ex, ab = oracle.matmul_exact(t, raw, X[8].cpu().numpy(), rows, dim1)
+        assert_dots(got[2][8].cpu().numpy(), ex, ab, "token 8")
+        w.free()
+    finally:
+        torch.cuda.synchronize()
+        c.close()
+
+
 def _no_subnormals(t, raw):
     """F16 weights without subnormals: the vector path reads them as 0
     (F16FloatTensor.kt:59-61), the exact sum does not."""

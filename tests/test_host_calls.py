@@ -219,3 +219,52 @@ def test_an_eager_call_leaves_the_scratch_for_its_capture(hip, t, m, rows, cols)
         assert p.batch(t, m, rows, cols) == ["k_tok_q4k" if t == Q4_K else "k_mat", "k_tok_reduce"]
         assert not [l for l in p.log() if l[0] == "malloc"]
         hip.stub_capture(s, 0)
+
+
+# several tokens on rows of more than 2048 columns: 16-token tiles with column splits
+WIDE = [(Q8_0, 12, 2048, 8192), (Q5_K, 40, 4096, 4096), (BF16, 4096, 8192, 8192), (F16, 5, 2048, 8192)]
+
+
+@pytest.mark.parametrize("t,m,rows,cols", WIDE)
+def test_wide_calls_on_several_streams_are_ordered(hip, t, m, rows, cols):
+    """Their split sums are in no memory that another stream's call, or a graph, may
+    be using."""
+    with Program(hip) as p:
+        streams = [None, p.stream(), p.stream()]
+        for k in (0, 1, 2, 2, 0, 1):
+            p.use(streams[k])
+            assert p.batch(t, m, rows, cols)[:2] == ["k_mat", "k_tok_reduce"]
+        p.assert_ordered()
+        used = {l[3] for l in p.log() if l[0] == "launch"}
+        # (captured: in the scratch)
+        p.use(streams[1])
+        hip.stub_capture(streams[1], 1)
+        hip.stub_clear()
+        assert p.batch(t, m, rows, cols)[:2] == ["k_mat", "k_tok_reduce"]
+        assert not used & {l[3] for l in p.log() if l[0] == "launch"}
+        hip.stub_capture(streams[1], 0)
+
+
+@pytest.mark.parametrize("t,m,rows,cols", WIDE)
+def test_wide_call_without_memory_for_its_split_sums(hip, t, m, rows, cols):
+    with Program(hip) as p:
+        p.batch(t, 2, rows, cols)  # (uploads)
+        hip.stub_free_bytes(100 << 10)
+        assert p.batch(t, m, rows, cols)[0] in ("k_rows", "k_wide")
+        assert hip.stub_last_error() == 0
+        s = p.stream()
+        p.use(s)
+        hip.stub_capture(s, 1)
+        assert p.batch(t, m, rows, cols)[0] in ("k_rows", "k_wide")
+        hip.stub_capture(s, 0)
+
+
+@pytest.mark.parametrize("t", [Q5_K, BF16, Q8_0])
+def test_split_sums_are_bounded(hip, t):
+    """4096 tokens x 8192 x 8192: the sums of four splits at once would be 512 MB, in
+    the workspace and again in the scratch."""
+    with Program(hip) as p:
+        p.batch(t, 2, 8192, 8192)
+        hip.stub_clear()
+        assert p.batch(t, 4096, 8192, 8192).count("k_tok_reduce") >= 8
+        assert sum(int(l[1]) for l in p.log() if l[0] == "malloc") <= 2 * (130 << 20)
