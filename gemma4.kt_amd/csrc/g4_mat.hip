@@ -28,7 +28,8 @@
 //   Q6_K     24.6 -> 14.6  53.8 -> 20.1  141.8 -> 32.9
 //   BF16     32.5 -> 10.4  90.3 -> 11.8  227.6 -> 16.6  1786 -> 98.5
 //   F16      39.5 -> 16.4 100.7 -> 20.8  245.1 -> 32.0
-// and against 64 bits the error falls from 1.2e-7..3.0e-7 to 1.0e-7..1.4e-7.
+// and against 64 bits the error falls from 1.2e-7..3.0e-7 to 0.7e-7..1.5e-7 (512 to
+// 32768 columns).
 #include "g4_mmfmt.hpp"
 #include "g4_internal.hpp"
 
@@ -192,7 +193,10 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
       const u32x4 u0 = *(const u32x4 *)p, u1 = *(const u32x4 *)(p + (SPB == 2 ? 16 : 4));
       float v[8];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = __uint_as_float(u0[k]), v[4 + k] = __uint_as_float(u1[k]);
+      for (int k = 0; k < 4; ++k) {
+        v[k] = __uint_as_float(u0[k]), v[4 + k] = __uint_as_float(u1[k]);
+        if (b & 1) v[k] = -v[k], v[4 + k] = -v[4 + k];  // (see the block sums)
+      }
       split3<false>(v, A[b][0], A[b][1], A[b][2]);
     }
   }
@@ -255,22 +259,25 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
             P[b][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[b][p], B[b], P[b][0], 0, 0, 0);
           }
         }
+      // Odd blocks multiply -x: the matrix cores round every sum down, which long rows
+      // would add up to more than the sums' other errors.
       if constexpr (HALF)
-        acc = (P[0][0] + P[1][0]) + (P[2][0] + P[3][0]);
+        acc = (P[0][0] - P[1][0]) + (P[2][0] - P[3][0]);
       else
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         f32x4 S;
         if constexpr (MIN) S = *(const f32x4 *)(wx + 16 * b + 4 * j);
+        const float sign = b & 1 ? -1.f : 1.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           if constexpr (SPB == 2) {
-            acc[i] = __builtin_fmaf(sc[b >> 1][2 * (b & 1)], P[b][0][i], acc[i]);
-            acc[i] = __builtin_fmaf(sc[b >> 1][2 * (b & 1) + 1], P[b][1][i], acc[i]);
+            acc[i] = __builtin_fmaf(sign * sc[b >> 1][2 * (b & 1)], P[b][0][i], acc[i]);
+            acc[i] = __builtin_fmaf(sign * sc[b >> 1][2 * (b & 1) + 1], P[b][1][i], acc[i]);
           } else if constexpr (MIN) {
-            acc[i] += rounded(sc[0][b] * P[b][0][i]) - rounded(of[b] * S[i]);
+            acc[i] += sign * (rounded(sc[0][b] * P[b][0][i]) - rounded(of[b] * S[i]));
           } else if constexpr (SPB == 1) {
-            acc[i] = __builtin_fmaf(sc[0][b], P[b][0][i], acc[i]);
+            acc[i] = __builtin_fmaf(sign * sc[0][b], P[b][0][i], acc[i]);
           }
         }
       }

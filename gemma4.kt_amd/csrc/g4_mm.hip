@@ -31,7 +31,10 @@ constexpr int MM_STAGE_FRAGS = 12;  // a 32-token tile's stage: 4 x 16 columns x
 // Operand (t, s, k, p) -- tokens 32 t .. 32 t + 31, columns 64 s + 16 k .. + 15,
 // part p -- is 1 KB at ((t * stages + s) * 12 + 3 k + p) * 1024: lane l's 16
 // bytes hold token l % 32, columns 8 (l / 32) .. + 7.  Tokens past M and columns
-// past dim1 are zeros.  sums[block][token]: the sum over 32 columns.
+// past dim1 are zeros.  sums[block][token]: the sum over 32 columns.  The second
+// block of each stage holds -x: the matrix cores round every sum down, which long
+// rows would add up to more than the sums' other errors; k_mm subtracts that
+// block's sums.
 //
 // A wave splits 16 columns of 32 tokens, eight per lane, and stores three whole
 // operands; a workgroup one stage of a token tile.  Bound by the latency of its
@@ -47,6 +50,7 @@ __global__ __launch_bounds__(256) void k_split(const float *x, int64_t x_stride,
   const u32x4a4 *src = (const u32x4a4 *)(x + (live ? (int64_t)tok * x_stride + col : 0));
   u32x4a4 u0 = src[0], u1 = src[1];
   if (!live) u0 = u1 = u32x4a4{0u, 0u, 0u, 0u};
+  if (k >= 2) u0 ^= 0x80000000u, u1 ^= 0x80000000u;  // the stage's second block
   const float v[8] = {__uint_as_float(u0.x), __uint_as_float(u0.y), __uint_as_float(u0.z), __uint_as_float(u0.w),
                       __uint_as_float(u1.x), __uint_as_float(u1.y), __uint_as_float(u1.z), __uint_as_float(u1.w)};
   // (an infinite x leaves NaN parts: the outputs it reaches are NaN and formed again by k_mm)
@@ -494,7 +498,7 @@ __global__ __launch_bounds__(MM_THREADS) void k_mm(MmArgs a) {
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const float sum = got[t][v] + (kh ? acc[t][1][v] : acc[t][0][v]);
+      const float sum = kh ? got[t][v] - acc[t][1][v] : acc[t][0][v] - got[t][v];
       const int tok = (t_base + 2 * wm + t) * 32 + 8 * (v >> 2) + 4 * j + (v & 3);
       if (tok < a.M && row < a.rows) {
         out[(int64_t)tok * a.y_stride + row] = sum;
@@ -537,7 +541,7 @@ MmPlan mm_plan(int type, int32_t M, int32_t rows, int32_t dim1, const DevInfo &d
   // Block sums follow one another in each accumulator, one per stage.  Up to 32
   // keep the error of the K-quants below that of the one-token kernels, up to 16
   // that of the other formats, whose kernels start from a smaller one (against 64
-  // bits, 2048 columns: Q4_K 1.6e-7 here, 1.9e-7 there; Q8_0 1.2e-7 there).
+  // bits, 2048 columns: Q4_K 1.5e-7 here, 2.0e-7 there; Q8_0 0.9e-7 and 1.2e-7).
   const int chain = type == T_Q4_K || type == T_Q6_K ? 32 : 16;
   const int smin = (p.stages + chain - 1) / chain, smax = std::min(std::max(smin, 16), p.stages);
   double best_us = 0;
@@ -610,8 +614,8 @@ bool mm_ok(int type, const TokArgs &a, const DevInfo &dev) {
   if (a.dim1 % unit != 0 || a.base % unit != 0 || a.row_stride % unit != 0) return false;
   switch (type) {
     case T_Q8_0: case T_Q4_0: case T_Q4_K: case T_Q6_K: return mm_faster(type, a, dev);
-    // F16's one-token kernels start from a smaller error, and the many splits of
-    // longer rows would go past it (as BF16's, which gains little: 512 tokens 97 / 76 us)
+    // F16 where its error is known to stay below the one-token kernels' (0.9e-7, 1.2e-7
+    // there); BF16 gains little (512 tokens 97 / 76 us)
     case T_F16: return a.dim1 <= 2048 && mm_faster(type, a, dev);
     default: return false;
   }

@@ -578,8 +578,10 @@ __global__ __launch_bounds__(WPB * 64) void k_tok_q4k(TokArgs a) {
   }
 }
 
-// y[m * y_stride + r] = sum over the column splits, in split order, of their
-// partial sums.  Thread t of workgroup (bx, m) covers V consecutive rows from
+// y[m * y_stride + r] = sum over the column splits of their partial sums: the first
+// nine in split order, then eight at a time (32 splits one after the other would
+// round more than the row engine does: 1.37e-7 against 1.35e-7 from 64 bits for
+// Q8_0 rows of 32768 columns, 1.11e-7 so).  Thread t of workgroup (bx, m) covers V consecutive rows from
 // V * (256 bx + t) of token m; the loads of up to 8 splits are all in flight
 // before the first add.
 template <int V>
@@ -594,9 +596,12 @@ __global__ __launch_bounds__(256) void k_tok_reduce(const float *part, int split
     fv v[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = *(const fv *)(part + (int64_t)min(k0 + k, splits - 1) * n + i);
+    fv t = k0 == 1 ? s : v[0];
+    if (k0 == 1) t += v[0];
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (k0 + k < splits) s += v[k];
+    for (int k = 1; k < 8; ++k)
+      if (k0 + k < splits) t += v[k];
+    s = k0 == 1 ? t : s + t;
   }
   *(fv *)(y + (int64_t)m * y_stride + r) = s;
 }

@@ -1039,6 +1039,31 @@ def test_batched_wide_rows_in_passes(g4, ctx, oracle):
     w.free()
 
 
+@pytest.mark.parametrize("t,m,rows,dim1", [(Q8_0, 16, 256, 16384), (Q8_0, 16, 256, 32768), (F16, 16, 256, 16384),
+                                           (BF16, 16, 256, 16384), (BF16, 16, 512, 8192), (Q8_0, 512, 512, 32768),
+                                           (Q4_0, 300, 2048, 8192), (Q6_K, 512, 8192, 2048)])
+def test_batched_error_not_above_one_token_calls(g4, ctx, oracle, t, m, rows, dim1):
+    """The 2-norm of a batched call's error against the exact sums is no larger than
+    that of one call per token on the same rows, with block scales of one sign, where
+    a one-sided rounding of every sum would add up."""
+    announce("batched error type %d M=%d %d x %d" % (t, m, rows, dim1))
+    raw = _no_subnormals(t, synth.weights(65, "me%d.%d" % (t, dim1), t, rows * dim1)).copy()
+    if t in (Q8_0, Q4_0):
+        raw.reshape(-1, 34 if t == Q8_0 else 18)[:, 1] &= 0x7F  # d >= 0
+    X = synth.activations(65, "mex%d.%d" % (m, dim1), m * dim1).reshape(m, dim1)
+    w = upload(g4, ctx, t, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    eb = e1 = 0.0
+    y = np.empty(rows, np.float32)
+    for i in range(0, m, max(1, m // 16)):
+        ex, _ = oracle.matmul_exact(t, raw, X[i], rows, dim1)
+        w.matmul(X[i], y, rows, dim1)
+        eb += float(np.sum((Y[i] - ex) ** 2))
+        e1 += float(np.sum((y - ex) ** 2))
+    assert eb <= e1, (eb / e1) ** 0.5
+    w.free()
+
+
 @pytest.mark.parametrize("t", [Q8_0, BF16])
 def test_batched_wide_rows_streams(g4, oracle, t):
     """Calls with column splits on two streams in turn, with no synchronisation
