@@ -353,26 +353,34 @@ bool mat_ok(int type, const TokArgs &a) {
   }
 }
 
-// A launch takes about 4 us (512 columns) to 7 us (2048) before its first tile, so
-// few tokens of a small matrix are faster on the row engine.  Measured, us, row
-// engine / here:
-//   8192 x 2048       3 tokens     4           5           8
-//     Q8_0          10.0 / 9.7   10.5 / 9.5  12.8 / 9.5  15.7 / 9.9
-//     Q4_0           7.7 / 8.7    8.8 / 8.7  10.4 / 8.7  13.3 / 9.0
-//     Q6_K          13.7 / 14.2  15.3 / 14.2 20.4 / 14.2 24.6 / 14.6
-//     BF16          17.1 / 9.9   18.9 / 10.0 24.9 / 10.2 32.5 / 10.4
-//   2048 x 8192 (column splits and their sum)
-//     Q8_0          10.1 / 11.9  11.8 / 12.0 13.6 / 12.0 18.6 / 12.3
-//     Q4_0           8.0 / 11.0   9.4 / 11.2 10.9 / 11.1 15.3 / 11.5
-//   2048 x 2048
-//     Q8_0           5.3 / 6.8    5.0 / 6.8   6.4 / 6.8   6.5 / 7.1
-//     Q6_K           6.0 / 9.8    6.2 / 9.8   7.7 / 9.9   8.7 / 9.9
-//     BF16           8.9 / 6.2    7.4 / 6.3   9.7 / 6.4  11.5 / 6.4
-// F16 (8192 x 2048, 3 tokens: 21.4 / 16.2) goes with BF16, Q5_K with the others.
+// A launch takes 4 us (512 columns) to 10 us (column splits) before its first tile;
+// the row engine takes about as little for its first round of waves and jumps where
+// M * rows starts the next one (16384 outputs of up to 4096 columns in the 32- and
+// 256-weight blocks).  So the line is a number of outputs, and a fewest M below which
+// the row engine's segments are as fast on any matrix.  Measured, us, row engine /
+// here, on either side of the line:
+//   Q8_0   1024 x 512,  8 tokens  3.2 / 3.7     2048 x 512,  5   4.3 / 3.8
+//          1024 x 2048, 16        5.8 / 7.3     17               7.4 / 7.3
+//          4096 x 2048, 4         6.1 / 6.8     5                9.5 / 6.8
+//          1024 x 8192, 8         9.5 / 9.6     9               11.1 / 10.1
+//   Q4_0   2048 x 2048, 12        6.3 / 6.7     14               8.2 / 6.8
+//          4096 x 4096, 6         9.8 / 10.3    7               11.5 / 10.3
+//   Q5_K   1024 x 2048, 16        6.8 / 8.2     17               8.7 / 8.4
+//   Q6_K   1024 x 2048, 16        8.1 / 9.9     17              10.6 / 10.4
+//   BF16   1024 x 2048, 4         5.6 / 5.7     5                8.0 / 5.7
+//          512 x 8192, 4          7.5 / 8.3     5               11.0 / 8.3
+//   F16    1024 x 2048, 4         7.1 / 8.8     5               12.3 / 8.7
+// Over 760 shapes a type (256 to 16384 rows, 512 to 8192 columns, 3 to 64 tokens) the
+// route taken is never more than 3.2% slower than the row engine.
 int32_t mat_min_tokens(int type, const TokArgs &a) {
-  if (type == T_BF16 || type == T_F16) return 3;
-  if ((int64_t)a.rows * a.dim1 < (8 << 20)) return 9;
-  return a.dim1 > 16 * MAT_COLS ? 6 : 4;
+  int64_t outputs;
+  if (type == T_BF16 || type == T_F16)
+    outputs = a.dim1 <= 2048 ? 4096 : a.dim1 <= 4096 ? 4608 : 2048;
+  else if (type == T_Q4_0)
+    outputs = a.dim1 <= 512 ? 8192 : a.dim1 <= 1024 ? 16384 : a.dim1 <= 4096 ? 24576 : 12288;
+  else
+    outputs = a.dim1 <= 512 ? 8192 : a.dim1 <= 4096 ? 16384 : type == T_Q6_K ? 4608 : 8192;
+  return (int32_t)std::max<int64_t>(type == T_BF16 || type == T_F16 ? 3 : 5, outputs / a.rows + 1);
 }
 
 // Tokens per pass: as many as MAT_PART_FLOATS holds the column splits' sums of.

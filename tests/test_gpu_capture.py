@@ -266,7 +266,7 @@ def test_batched_wide_rows_captured(g4, reserve):
     segment of the row engine per token) instead of failing; with it the replays
     give the eager bits."""
     announce("capture: batched wide rows, %d bytes reserved" % reserve)
-    m, rows, cols = 12, 40, 4096
+    m, rows, cols = 12, 1401, 4096
     raw = synth.weights(46, "bw", 8, rows * cols)
     X = torch.from_numpy(synth.activations(46, "bwx", m * cols).reshape(m, cols)).cuda()
     Y = torch.empty((m, rows), device="cuda")

@@ -997,26 +997,32 @@ def test_moe_route_edge_cases(g4, ctx, oracle, case):
 # in the last slice (columns 32, 64 and 96 past a multiple of 128), workgroups of
 # 4, 8 and 16 waves with slices to spare, column splits (2176 and 8192 columns),
 # rows behind an offset, one to three token tiles, and enough rows that a
-# workgroup walks several tiles.  BF16 and F16 take this route from three tokens
-# on, the others here from nine.
-MAT_SHAPES = [(9, 17, 512, 0), (16, 33, 1024, 1), (17, 40, 2048, 0), (33, 50, 1152, 2), (40, 24, 2176, 0),
-              (9, 20, 8192, 0), (64, 4500, 256, 0)]
+# workgroup walks several tiles.  (tests/test_host_calls.py checks that these take
+# k_mat; calls of few outputs stay on the row engine.)
+MAT_SHAPES = [(9, 921, 512, 0), (16, 1041, 1024, 1), (17, 1464, 2048, 0), (33, 754, 1152, 2), (40, 632, 2176, 0),
+              (9, 1381, 8192, 0), (64, 4500, 256, 0)]
+MAT_ODD_BLOCKS = [(9, 932, 32, 0), (9, 1827, 544, 1), (20, 1234, 1056, 0), (11, 2242, 2144, 3)]
+MAT_FEW = [(BF16, 3, 1400, 64), (F16, 3, 1393, 192), (BF16, 5, 930, 2112), (Q8_0, 5, 8192, 1024), (Q4_0, 7, 4096, 4096),
+           (Q6_K, 5, 4096, 2048)]
+ROW_SHAPES = [(9, 17, 512, 0), (16, 33, 1024, 1), (17, 40, 2048, 0), (33, 50, 1152, 2), (40, 24, 2176, 0),
+              (9, 20, 8192, 0)]
 
 
 @pytest.mark.parametrize("t", [Q8_0, Q4_0, Q5_K, Q6_K, BF16, F16])
-@pytest.mark.parametrize("m,rows,dim1,off_rows", MAT_SHAPES)
+@pytest.mark.parametrize("m,rows,dim1,off_rows", MAT_SHAPES + ROW_SHAPES)
 def test_batched_matrix_core_shapes(g4, ctx, oracle, t, m, rows, dim1, off_rows):
     _batched_case(g4, ctx, oracle, t, m, rows, dim1, off_rows)
 
 
 @pytest.mark.parametrize("t", [Q8_0, Q4_0])
-@pytest.mark.parametrize("m,rows,dim1,off_rows", [(9, 20, 32, 0), (9, 35, 544, 1), (20, 18, 1056, 0), (11, 16, 2144, 3)])
+@pytest.mark.parametrize("m,rows,dim1,off_rows", MAT_ODD_BLOCKS + [(9, 20, 32, 0), (9, 35, 544, 1), (20, 18, 1056, 0),
+                                                                   (11, 16, 2144, 3)])
 def test_batched_matrix_core_odd_blocks(g4, ctx, oracle, t, m, rows, dim1, off_rows):
     _batched_case(g4, ctx, oracle, t, m, rows, dim1, off_rows)
 
 
-@pytest.mark.parametrize("t,m,rows,dim1", [(BF16, 3, 40, 64), (F16, 3, 33, 192), (BF16, 5, 20, 2112),
-                                           (Q8_0, 4, 8192, 1024), (Q4_0, 6, 2048, 4096), (Q6_K, 4, 4096, 2048)])
+@pytest.mark.parametrize("t,m,rows,dim1", MAT_FEW + [(BF16, 3, 40, 64), (F16, 3, 33, 192), (BF16, 5, 20, 2112),
+                                                     (Q8_0, 4, 8192, 1024), (Q4_0, 6, 2048, 4096), (Q6_K, 4, 4096, 2048)])
 def test_batched_matrix_core_few_tokens(g4, ctx, oracle, t, m, rows, dim1):
     _batched_case(g4, ctx, oracle, t, m, rows, dim1, 0)
 
@@ -1039,7 +1045,7 @@ def test_batched_wide_rows_in_passes(g4, ctx, oracle):
     w.free()
 
 
-@pytest.mark.parametrize("t,m,rows,dim1", [(Q8_0, 16, 256, 16384), (Q8_0, 16, 256, 32768), (F16, 16, 256, 16384),
+@pytest.mark.parametrize("t,m,rows,dim1", [(Q8_0, 16, 544, 16384), (Q8_0, 16, 528, 32768), (F16, 16, 256, 16384),
                                            (BF16, 16, 256, 16384), (BF16, 16, 512, 8192), (Q8_0, 512, 512, 32768),
                                            (Q4_0, 300, 2048, 8192), (Q6_K, 512, 8192, 2048)])
 def test_batched_error_not_above_one_token_calls(g4, ctx, oracle, t, m, rows, dim1):
@@ -1128,7 +1134,7 @@ def test_batched_matrix_core_non_finite_and_wide_x(g4, ctx, oracle, t):
     the products w * x (NaN for w = 0, else of the infinity's sign); a token spanning
     1e-20..1e20 and the finite tokens that share the waves stay within the bound."""
     announce("batched non-finite x type %d" % t)
-    m, rows, dim1 = 12, 40, 2048
+    m, rows, dim1 = 12, 2056, 2048
     raw = _no_subnormals(t, synth.weights(62, "mtn%d" % t, t, rows * dim1))
     X = synth.activations(62, "mtnx", m * dim1).reshape(m, dim1)
     X[4] *= (10.0 ** np.random.default_rng(62).uniform(-20, 20, dim1)).astype(np.float32)
@@ -1149,7 +1155,7 @@ def test_batched_matrix_core_infinite_weight(g4, ctx, oracle):
     """An infinite BF16 weight gives its row infinite outputs (not the NaN that an
     infinity times an activation's zero residual part would)."""
     announce("batched infinite bf16 weight")
-    m, rows, dim1 = 5, 20, 512
+    m, rows, dim1 = 5, 840, 512
     raw = synth.weights(63, "mti", BF16, rows * dim1).copy()
     raw.view(np.uint16)[3 * dim1 + 100] = 0x7F80
     X = np.ones((m, dim1), np.float32)
@@ -1317,7 +1323,7 @@ def test_batched_many_tokens_after_their_stream_is_gone(g4):
         c.close()
 
 
-@pytest.mark.parametrize("m,rows,dim1", [(5, 20, 512), (512, 8192, 1024)])
+@pytest.mark.parametrize("m,rows,dim1", [(5, 840, 512), (512, 8192, 1024)])
 def test_batched_f16_exponent_31(g4, ctx, oracle, m, rows, dim1):
     """F16 exponent 31 is the finite 2^16 * 1.m in the vector path
     (F16FloatTensor.kt:59-61): rows with such weights get the one-token call's finite

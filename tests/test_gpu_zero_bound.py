@@ -199,7 +199,7 @@ def test_zero_rows_batched_many(g4, ctx, oracle, t):
     """20 tokens of the formats other than Q4_K take their own matrix-core kernel:
     Q4_0's integers are 0 where the weight is, Q5_K's two sums run alike."""
     announce("zero-bound batched type %d M=20" % t)
-    rows, cols, m = 96, 2048, 20
+    rows, cols, m = 1248, 2048, 20
     kinds = _kinds(rows)
     raw = BUILD[t](rows, cols, kinds)
     X = synth.activations(8, "X%d" % m, m * cols).reshape(m, cols)

@@ -13,6 +13,7 @@ import pytest
 
 import build as pkg_build
 import g4hip
+import test_gpu_parity as gpu
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 Q8_0, Q4_0, Q4_K, Q5_K, Q6_K, F16, BF16 = 8, 2, 12, 13, 14, 1, 30
@@ -268,3 +269,34 @@ def test_split_sums_are_bounded(hip, t):
         hip.stub_clear()
         assert p.batch(t, 4096, 8192, 8192).count("k_tok_reduce") >= 8
         assert sum(int(l[1]) for l in p.log() if l[0] == "malloc") <= 2 * (130 << 20)
+
+
+MAT_TYPES = [Q8_0, Q4_0, Q5_K, Q6_K, BF16, F16]
+
+
+def test_shapes_meant_for_the_16_token_tiles_take_them(hip):
+    """The sizes at which tests/test_gpu_parity.py and its neighbours test k_mat."""
+    with Program(hip) as p:
+        cases = [(t,) + s[:3] for t in MAT_TYPES for s in gpu.MAT_SHAPES]
+        cases += [(t,) + s[:3] for t in (Q8_0, Q4_0) for s in gpu.MAT_ODD_BLOCKS] + gpu.MAT_FEW
+        cases += [(t, 12, 2056, 2048) for t in MAT_TYPES]
+        cases += [(BF16, 5, 840, 512), (F16, 5, 840, 512), (BF16, 700, 8192, 4160), (Q8_0, 12, 1401, 4096)]
+        cases += [(t, m, 2048, 8192) for t in (Q8_0, BF16) for m in (9, 12, 64)]
+        cases += [(t, 20, 1248, 2048) for t in (Q4_0, Q5_K)]
+        cases += [(Q8_0, 16, 544, 16384), (Q8_0, 16, 528, 32768), (F16, 16, 256, 16384), (BF16, 16, 256, 16384),
+                  (BF16, 16, 512, 8192)]
+        for c in cases:
+            assert p.batch(*c)[0] == "k_mat", c
+
+
+# (type, tokens, rows, columns), just below and above the outputs from which the
+# 16-token tiles are the faster route; the measured times stand at mat_min_tokens
+@pytest.mark.parametrize("t,m,rows,cols", [(Q8_0, 8, 1024, 512), (Q8_0, 32, 512, 4096), (Q8_0, 16, 1024, 2048),
+                                           (Q8_0, 4, 4096, 2048), (Q8_0, 8, 1024, 8192), (Q4_0, 12, 2048, 2048),
+                                           (Q4_0, 6, 4096, 4096), (Q5_K, 16, 1024, 2048), (Q6_K, 16, 1024, 2048),
+                                           (Q6_K, 9, 512, 8192), (BF16, 4, 1024, 2048), (F16, 4, 1024, 2048),
+                                           (BF16, 4, 512, 8192), (BF16, 9, 512, 3072)])
+def test_few_outputs_stay_on_the_row_engine(hip, t, m, rows, cols):
+    with Program(hip) as p:
+        assert p.batch(t, m, rows, cols)[0] in ("k_rows", "k_wide")
+        assert p.batch(t, m + 1 + (t == Q4_0), rows, cols)[0] == "k_mat"
