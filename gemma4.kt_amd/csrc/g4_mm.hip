@@ -588,6 +588,9 @@ hipError_t mm_launch(const MmArgs &a, hipStream_t s) {
 //   Q6_K  8192 x 2048     53.6 / 33.1  93 / 46.1  140 / 65.5  203 / 70.9
 //   F16   8192 x 2048     63.2 / 37.0 116 / 56.8  169 / 96.8  249 / 110 (f16_parts since faster: 54.2, 111 here)
 //   Q8_0  2048 x 2048     13.1 / 22.7  20 / 24.8   27 / 29.2   38 / 31.4
+// Q4_K over 408 shapes of 65 to 1024 tokens, 512 to 16384 rows and 512 to 8192
+// columns: never more than 3% slower than k_tok_q4k (4096 x 512, 256 tokens 17.6 /
+// 24.5; 5000 x 1024, 320 tokens 26.6 / 31.7; 16384 x 512, 512 tokens 106 / 42.8).
 static bool mm_faster(int type, const TokArgs &a, const DevInfo &dev) {
   if (a.M <= 64) return false;
   const int32_t M = std::min<int32_t>(a.M, 1024);
@@ -595,7 +598,8 @@ static bool mm_faster(int type, const TokArgs &a, const DevInfo &dev) {
   switch (type) {
     case T_Q8_0: tile = 1.95; break;
     case T_Q4_0: tile = 1.5; break;
-    case T_Q4_K: tile = 1.1; break;
+    // (of 1024 columns and fewer, half of the waves or more have none)
+    case T_Q4_K: tile = a.dim1 <= 1024 ? 0.78 : 1.1; break;
     default: tile = 3.1; break;  // Q6_K, F16
   }
   const int n_sl = (a.dim1 + 127) / 128, splits = (n_sl + 15) / 16, sps = (n_sl + splits - 1) / splits;

@@ -300,3 +300,12 @@ def test_few_outputs_stay_on_the_row_engine(hip, t, m, rows, cols):
     with Program(hip) as p:
         assert p.batch(t, m, rows, cols)[0] in ("k_rows", "k_wide")
         assert p.batch(t, m + 1 + (t == Q4_0), rows, cols)[0] == "k_mat"
+
+
+@pytest.mark.parametrize("m,rows,cols", [(256, 4096, 512), (128, 8192, 512), (200, 8192, 1024), (200, 5000, 512),
+                                         (400, 4096, 1024)])
+def test_short_q4_k_rows_stay_on_the_16_token_tiles(hip, m, rows, cols):
+    """Where the tiled product takes 22 to 39% longer."""
+    with Program(hip) as p:
+        assert p.batch(Q4_K, m, rows, cols) == ["k_tok_q4k"]
+        assert "k_mm" in p.batch(Q4_K, 4 * m, rows, cols)
