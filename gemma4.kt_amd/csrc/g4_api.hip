@@ -632,6 +632,7 @@ int moe_dev(g4_ctx *ctx, const g4_weight *wgu, const g4_weight *wdn, int32_t n_e
     dn.y = d_ys;
     dn.y_stride = dim;
     if (g4::moe_grp_ok(wgu->type, true, gu) && g4::moe_grp_ok(wdn->type, false, dn) && n_experts < 65535 &&
+        g4::moe_grp_faster(gu, dn, ctx->dev) &&
         (!route || route->n_experts <= g4::ROUTE_LAUNCH_MAX_E)) {
       if (route)
         G4_TRY(launch_status(g4::launch_route(route->d_logits, T, route->n_experts, k, route->renormalize,

@@ -142,6 +142,9 @@ struct MoeGrpArgs {
   float *gu;
 };
 bool moe_grp_ok(int type, bool gate_up, const MoeGrpArgs &a);
+// Whether a call's two grouped launches (gu.S pairs, gu.x_div slots a token) are the
+// faster route.
+bool moe_grp_faster(const MoeGrpArgs &gu, const MoeGrpArgs &dn, const DevInfo &dev);
 // Grants the grouped kernels their largest dynamic LDS size on the current
 // device; called once per device before any launch (g4_open).
 hipError_t moe_grp_init_device();

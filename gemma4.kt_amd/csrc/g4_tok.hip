@@ -47,6 +47,7 @@
 #include "g4_internal.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace g4 {
@@ -1333,6 +1334,25 @@ bool moe_grp_ok(int type, bool gate_up, const MoeGrpArgs &a) {
   if (a.base0 % 128 != 0 || a.base1 % 128 != 0 || a.row_stride % 128 != 0 || a.expert_stride % 128 != 0)
     return false;
   return a.S >= 1 && a.rows >= 1 && a.x_div >= 1 && a.n_experts >= 1;
+}
+
+// Whole 128-column slices: always, of the calls that come here (MOE_GROUPED_MIN_T).
+// Other rows of 64-column groups have slower tiles and, per pair, the faster kernels:
+// the estimates below (us; uniform routing) are within 20% of the measured times of
+// 3600 grouped and 1440 per-pair calls: 41 to 256 tokens, 1 to 8 slots, 16 to 256
+// experts, 512 to 2048 columns, ff 192 to 1728.  Grouped / per pair, measured:
+//   128 experts, 1024 columns, ff 704   41 tokens x 4 slots  103 / 48    256 x 8  173 / 352
+//   32 experts,  2048 columns, ff 704   41 x 4                68 / 84    256 x 8  213 / 668
+//   300 experts, 512 columns,  ff 320   41 x 8               102 / 49    256 x 8  150 / 171
+// Grouped only where the estimate is 15% lower: of 3600 calls five are then slower
+// than per pair by more than 3% (the worst by 17%).
+bool moe_grp_faster(const MoeGrpArgs &gu, const MoeGrpArgs &dn, const DevInfo &dev) {
+  if (gu.dim1 % 128 == 0 && dn.dim1 % 128 == 0) return true;
+  const double S = gu.S, E = gu.n_experts, dim = gu.dim1, ff = dn.dim1;
+  const double passes = E * (1.0 - std::exp(-S / E)) + std::max(0.0, S / 16.0 - E / 2.0);
+  const double grouped = 32.0 + 1.32 * passes * (2.0 * ff + dim) / (16.0 * dev.cu_count) + 1.67e-6 * S * (ff + dim);
+  const double per_pair = 16.0 + (dim > 1024 ? 1.3e-3 * ff * S / gu.x_div : 0.0) + S * (6.4e-5 * dim + 1.6e-4 * ff);
+  return 1.15 * grouped < per_pair;
 }
 
 hipError_t moe_grp_init_device() {

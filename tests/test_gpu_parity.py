@@ -1170,10 +1170,14 @@ def test_batched_matrix_core_infinite_weight(g4, ctx, oracle):
 # more passes than workgroups (300 experts, some hit twice over), a pass shared by
 # several (one expert: its 24 tiles on as many workgroups), stretches that end
 # within a pass (90 passes over 256 CUs) and span two, an expert with most of the
-# pairs, pairs of no expert, and down rows that start on a 64-column group (320).
-@pytest.mark.parametrize("E,D,FF,K,T,skew,drop", [(300, 256, 128, 8, 120, 0, 0), (1, 512, 192, 1, 50, 0, 0),
-                                                   (90, 256, 320, 2, 60, 0, 0), (24, 256, 128, 4, 100, 60, 7),
-                                                   (16, 128, 64, 2, 45, 0, 45)])
+# pairs, pairs of no expert, and down rows that start on a 64-column group (320) in
+# a call large enough to run grouped with them.
+MOE_STRETCHES = [(300, 256, 128, 8, 120, 0, 0), (90, 256, 384, 2, 60, 0, 0), (24, 256, 128, 4, 100, 60, 7),
+                 (16, 128, 128, 2, 45, 0, 45), (1, 512, 128, 1, 50, 0, 0), (6, 256, 320, 4, 500, 90, 11)]
+
+
+@pytest.mark.parametrize("E,D,FF,K,T,skew,drop", MOE_STRETCHES + [(1, 512, 192, 1, 50, 0, 0), (90, 256, 320, 2, 60, 0, 0),
+                                                                  (16, 128, 64, 2, 45, 0, 45)])
 def test_moe_grouped_equal_stretches(g4, ctx, oracle, E, D, FF, K, T, skew, drop):
     announce("moe grouped stretches E=%d D=%d FF=%d K=%d T=%d" % (E, D, FF, K, T))
     gu = synth.q4_k(66, "gu%d.%d" % (E, FF), E * 2 * FF * D)

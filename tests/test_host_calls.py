@@ -17,7 +17,7 @@ import test_gpu_parity as gpu
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 Q8_0, Q4_0, Q4_K, Q5_K, Q6_K, F16, BF16 = 8, 2, 12, 13, 14, 1, 30
-KERNELS = ["k_split", "k_mm", "k_tok_q4k", "k_tok_reduce", "k_mat", "k_rows", "k_wide"]
+KERNELS = ["k_split", "k_mm", "k_tok_q4k", "k_tok_reduce", "k_mat", "k_rows", "k_wide", "k_grp_q4k"]
 
 
 def _run(cmd):
@@ -81,18 +81,27 @@ class Program:
     def use(self, stream):
         assert self.hip.g4_ctx_set_stream(self.ctx, stream) == 0
 
+    def weight(self, t, elems):
+        if (t, elems) not in self.weights:
+            n, w = (ctypes.c_int64 * 1)(), (ctypes.c_void_p * 1)()
+            assert self.hip.g4_byte_size(t, elems, n) == 0
+            assert self.hip.g4_upload(self.ctx, t, ctypes.create_string_buffer(n[0]), n[0], elems, w) == 0
+            self.weights[t, elems] = w[0]
+        return self.weights[t, elems]
+
     def batch(self, t, m, rows, cols):
         """matmul_batch_dev; the names of the kernels it launched."""
-        key = (t, rows * cols)
-        if key not in self.weights:
-            n = (ctypes.c_int64 * 1)()
-            assert self.hip.g4_byte_size(t, rows * cols, n) == 0
-            w = (ctypes.c_void_p * 1)()
-            assert self.hip.g4_upload(self.ctx, t, ctypes.create_string_buffer(n[0]), n[0], rows * cols, w) == 0
-            w = w[0]
-            self.weights[key] = w
+        w = self.weight(t, rows * cols)
         before = len(self.log())
-        rc = self.hip.g4_matmul_batch_dev(self.ctx, self.weights[key], 0, 4096, m, 8192, rows, cols)
+        rc = self.hip.g4_matmul_batch_dev(self.ctx, w, 0, 4096, m, 8192, rows, cols)
+        assert rc == 0, self.hip.g4_last_error()
+        return [self.kernel(l[1]) for l in self.log()[before:] if l[0] == "launch"]
+
+    def moe(self, experts, dim, ff, k, tokens):
+        """moe_dev; the names of the kernels it launched."""
+        gu, dn = self.weight(Q4_K, experts * 2 * ff * dim), self.weight(Q4_K, experts * dim * ff)
+        before = len(self.log())
+        rc = self.hip.g4_moe_dev(self.ctx, gu, dn, 4096, tokens, dim, ff, 8192, 12288, k, 16384)
         assert rc == 0, self.hip.g4_last_error()
         return [self.kernel(l[1]) for l in self.log()[before:] if l[0] == "launch"]
 
@@ -309,3 +318,21 @@ def test_short_q4_k_rows_stay_on_the_16_token_tiles(hip, m, rows, cols):
     with Program(hip) as p:
         assert p.batch(Q4_K, m, rows, cols) == ["k_tok_q4k"]
         assert "k_mm" in p.batch(Q4_K, 4 * m, rows, cols)
+
+
+# (experts, columns, ff, slots, tokens)
+@pytest.mark.parametrize("shape,grouped", [((128, 1024, 704, 4, 41), False), ((128, 1024, 704, 8, 256), True),
+                                           ((32, 2048, 704, 8, 41), True), ((32, 2048, 704, 1, 256), True),
+                                           ((128, 2048, 704, 2, 64), False), ((300, 512, 320, 8, 41), False),
+                                           ((32, 1024, 320, 1, 256), False), ((32, 1024, 768, 1, 41), True),
+                                           ((32, 1024, 768, 8, 40), False)])
+def test_grouped_experts_where_they_are_faster(hip, shape, grouped):
+    """Both sides' measured times stand at moe_grp_faster."""
+    with Program(hip) as p:
+        assert ("k_grp_q4k" in p.moe(*shape)) == grouped
+
+
+def test_shapes_meant_for_the_grouped_experts_take_them(hip):
+    with Program(hip) as p:
+        for E, D, FF, K, T, *_ in gpu.MOE_STRETCHES:
+            assert p.moe(E, D, FF, K, T).count("k_grp_q4k") == 2, (E, D, FF)
