@@ -957,7 +957,7 @@ __global__ __launch_bounds__(MG_WPB * 64) void k_moe_grp(MoeGrpArgs a) {
 // three passes' x, and no CU waits for an expert with twice the pairs.  (Row blocks
 // x experts, each looping over its passes, left most CUs idle while the experts of
 // more than 16 pairs ran their second pass: 200 tokens, 128 experts, top-8,
-// 429 -> 271 us a call; 60 tokens, 32 experts, top-4, ff 704, 117 -> 71 us.)
+// 431 -> 264 us a call; 41 tokens, 32 experts, top-8, ff 704, 128 -> 69 us.)
 constexpr int GT_WPB = 16;
 constexpr int GT_MAX_E = GT_WPB * 64;  // experts: one thread each
 
@@ -983,12 +983,15 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
   const int ng = max(0, min(GPW, C - g0));      // wave-uniform
   const int n_rt = (a.rows + 15) >> 4;
 
-  // passes of expert tid, and those before it
-  for (int k = tid; k <= a.n_experts; k += WPB * 64) ecnt[k] = 0;
-  __syncthreads();
-  for (int p = tid; p < a.S; p += WPB * 64) {
-    const int id = a.ids[p];
-    atomicAdd(&ecnt[id >= 0 && id < a.n_experts ? id : a.n_experts], 1);
+  // passes of expert tid, and those before it (the first ids are read behind the zeros)
+  {
+    int id = tid < a.S ? a.ids[tid] : 0;
+    for (int k = tid; k <= a.n_experts; k += WPB * 64) ecnt[k] = 0;
+    __syncthreads();
+    for (int p = tid; p < a.S; p += WPB * 64) {
+      if (p != tid) id = a.ids[p];
+      atomicAdd(&ecnt[id >= 0 && id < a.n_experts ? id : a.n_experts], 1);
+    }
   }
   __syncthreads();
   const int np = tid < a.n_experts ? (ecnt[tid] + 15) >> 4 : 0;
@@ -1007,6 +1010,28 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
     all += wcnt[w];
   }
   const bool none = ecnt[a.n_experts] > 0;  // some pairs have no expert: their rows are zeros
+  // The stretch [u, u1) of units.  With fewer passes than workgroups, one pass (or
+  // a part of one) per workgroup where the longest part is no longer than an equal
+  // stretch and the start of the second pass in it (about five tiles' time: its
+  // pairs, their x and its split).
+  const int64_t units = (int64_t)all * n_rt;
+  const int parts = all > 0 ? (int)gridDim.x / all : 0, bx = (int)blockIdx.x;
+  int64_t u = units * bx / (int)gridDim.x, u1 = units * (bx + 1) / (int)gridDim.x;
+  if (parts > 0) {
+    const int len = (n_rt + parts - 1) / parts;
+    if (len <= units / (int)gridDim.x + 5) {
+      const int item = bx / parts, t0 = min(n_rt, bx % parts * len);
+      u = item < all ? (int64_t)item * n_rt + t0 : 0;
+      u1 = item < all ? (int64_t)item * n_rt + min(n_rt, t0 + len) : 0;
+    }
+  }
+  int item = (int)(u / n_rt), rt0 = (int)(u - (int64_t)item * n_rt), left = (int)(u1 - u);
+  // the item's expert and pass
+  auto find = [&](int first, int n) {
+    const int k = item - first;
+    if (k >= 0 && k < n) cur[0] = tid, cur[1] = k;
+  };
+  find(before - np, np);
   __syncthreads();  // ecnt and wcnt are reused
   if (tid < a.n_experts) ecnt[tid] = (before - np) << 13 | np;  // at most 4096 passes (MG_MAX_S)
   if (none)
@@ -1042,31 +1067,9 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
     __syncthreads();
   };
 
-  // The stretch [u, u1) of units.  With fewer passes than workgroups, one pass (or
-  // a part of one) per workgroup where the longest part is no longer than an equal
-  // stretch and the start of the second pass in it (about five tiles' time: its
-  // pairs, their x and its split).
-  const int64_t units = (int64_t)all * n_rt;
-  const int parts = all > 0 ? (int)gridDim.x / all : 0, bx = (int)blockIdx.x;
-  int64_t u = units * bx / (int)gridDim.x, u1 = units * (bx + 1) / (int)gridDim.x;
-  if (parts > 0) {
-    const int len = (n_rt + parts - 1) / parts;
-    if (len <= units / (int)gridDim.x + 5) {
-      const int item = bx / parts, t0 = min(n_rt, bx % parts * len);
-      u = item < all ? (int64_t)item * n_rt + t0 : 0;
-      u1 = item < all ? (int64_t)item * n_rt + min(n_rt, t0 + len) : 0;
-    }
-  }
-  while (u < u1) {
-    const int item = (int)(u / n_rt), rt0 = (int)(u - (int64_t)item * n_rt);
-    const int rt1 = (int)min((int64_t)n_rt, rt0 + (u1 - u));
-    u += rt1 - rt0;
-    __syncthreads();  // every wave is done with the previous pass's LDS
-    if (tid < a.n_experts) {
-      const int k = item - (ecnt[tid] >> 13);
-      if (k >= 0 && k < (ecnt[tid] & 0x1FFF)) cur[0] = tid, cur[1] = k;
-    }
-    __syncthreads();
+  while (left > 0) {
+    const int rt1 = min(n_rt, rt0 + left);
+    left -= rt1 - rt0;
     const int e = __builtin_amdgcn_readfirstlane(cur[0]);
     scan(e, __builtin_amdgcn_readfirstlane(cur[1]));
     const int64_t base = (int64_t)e * a.expert_stride + a.base0;
@@ -1313,6 +1316,13 @@ __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
         if (rt + 1 < rt1) tile(rt + 1, QB, HB, GB, [] {});
         __builtin_amdgcn_sched_barrier(0);
       }
+    }
+    if (left > 0) {
+      __syncthreads();  // every wave is done with the pass's LDS
+      ++item;
+      rt0 = 0;
+      if (tid < a.n_experts) find(ecnt[tid] >> 13, ecnt[tid] & 0x1FFF);
+      __syncthreads();
     }
   }
 }
