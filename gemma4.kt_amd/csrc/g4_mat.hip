@@ -42,18 +42,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int MAT_COLS = 128;  // columns per wave
 
-// The columns [c0, c1) of one dot product in fp32 from the decoded weights.  A
-// sum the matrix cores give as NaN -- an infinite or NaN activation or weight (an
-// infinity's residual parts are NaN), or block sums that overflowed with both
-// signs -- is formed again this way.
-template <int TYPE>
-G4_DEV float mat_plain_dot(const uint8_t *W, int64_t E, const float *x, int c0, int c1, int dim1) {
-  float s = 0.f;
-#pragma clang loop unroll(disable)
-  for (int c = c0; c < c1; ++c) s = __builtin_fmaf(dot_elem<TYPE>(W, E + c, c, dim1), x[c], s);
-  return s;
-}
-
 template <int TYPE>
 constexpr bool mat_half = TYPE == T_BF16 || TYPE == T_F16;
 
@@ -218,8 +206,9 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
 
   float *out = gridDim.y == 1 ? a.y : a.part + (int64_t)blockIdx.y * a.M * a.rows;
   const int64_t out_stride = gridDim.y == 1 ? a.y_stride : a.rows;
+  uint64_t bad = 0;
   for (int rt = rt0, buf = 0; rt < rt1; ++rt, buf ^= 1) {
-    bf16x8 B[4], L[TYPE == T_F16 ? 4 : 1];
+    bf16x8 B[4];
     f32x4 sc[SPB == 2 ? 2 : 1];
     f32x4 of = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -227,9 +216,6 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
 #pragma unroll
     for (int k = 0; k < SPB; ++k) sc[k] = *(const f32x4 *)(ws + n * 4 * SPB + 4 * k);
     if constexpr (MIN) of = *(const f32x4 *)(wo + n * 4);
-    if constexpr (TYPE == T_F16)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) f16_parts(__builtin_bit_cast(u32x4, B[b]), B[b], L[b]);
     __builtin_amdgcn_sched_barrier(0);
     load(min(rt + 1, rt1 - 1), wr);
     __builtin_amdgcn_sched_barrier(0);
@@ -241,6 +227,25 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
       for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int k = 0; k < (SPB == 2 ? 2 : 1); ++k) P[b][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (TYPE == T_F16) {
+        // (two blocks at a time: the parts of four would not fit the registers, 19
+        // tokens of 8192 x 2048 22.0 us, 15.8 so)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          if (g >= ng) continue;
+          bf16x8 H[2], L[2];
+#pragma unroll
+          for (int b = 0; b < 2; ++b) f16_parts(__builtin_bit_cast(u32x4, B[2 * g + b]), H[b], L[b]);
+#pragma unroll
+          for (int p = 2; p >= 0; --p)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+              f32x4 &c = P[2 * g + b][0];
+              c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[2 * g + b][p], L[b], c, 0, 0, 0);
+              c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[2 * g + b][p], H[b], c, 0, 0, 0);
+            }
+        }
+      } else
 #pragma unroll
       for (int p = 2; p >= 0; --p)
 #pragma unroll
@@ -255,7 +260,6 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
             for (int k = 0; k < 2; ++k)
               P[b][k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x2.h[k], w2.h[k], P[b][k], 0, 0, 0);
           } else {
-            if constexpr (TYPE == T_F16) P[b][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[b][p], L[b], P[b][0], 0, 0, 0);
             P[b][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[b][p], B[b], P[b][0], 0, 0, 0);
           }
         }
@@ -298,13 +302,30 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
         for (int w = 0; w < d; ++w) v[w] = v[2 * w] + v[2 * w + 1];
       float s = v[0];
       const int r = rt * 16 + n, m = 4 * j + wid;
-      if (r < a.rows && m < mt) {
-        if (redo<TYPE>(s))
-          s = mat_plain_dot<TYPE>(a.W, a.base + (int64_t)r * a.row_stride, a.x + (int64_t)(tok0 + m) * a.x_stride,
-                                  sl0 * MAT_COLS, min(a.dim1, (sl0 + nw) * MAT_COLS), a.dim1);
-        out[(int64_t)(tok0 + m) * out_stride + r] = s;
-      }
+      const bool mine = r < a.rows && m < mt;
+      if (mine) out[(int64_t)(tok0 + m) * out_stride + r] = s;
+      bad |= __builtin_amdgcn_ballot_w64(mine && redo<TYPE>(s));
     }
+  }
+  if (bad == 0) return;
+  // Waves 0..3: each lane reads its own outputs back, and the wave forms these again
+  // (here and not where they are stored: in the loop it would cost registers, 19
+  // tokens of Q8_0 14.2 -> 14.9 us, Q6_K 22.4 -> 25.3).
+  for (int rt = rt0; rt < rt1; ++rt) {
+    const int r = rt * 16 + n, m = 4 * j + wid;
+    const bool mine = r < a.rows && m < mt;
+    volatile float *o = out + (int64_t)(tok0 + (mine ? m : 0)) * out_stride + (mine ? r : 0);
+    float s = mine ? *o : 0.f;
+    const bool again = mine && redo<TYPE>(s);
+    const uint64_t todo = __builtin_amdgcn_ballot_w64(again);
+    for (int l0 = 0; l0 < 64; l0 += 16) {  // token 4 (l0 / 16) + wid
+      const uint64_t lanes = todo & (0xFFFFull << l0);
+      if (lanes)
+        form_again<TYPE>(a.W, a.base + (int64_t)(rt * 16) * a.row_stride, a.row_stride, l0, lanes,
+                         a.x + (int64_t)(tok0 + l0 / 4 + wid) * a.x_stride, sl0 * MAT_COLS,
+                         min(a.dim1, (sl0 + nw) * MAT_COLS), a.dim1, s);
+    }
+    if (again) *o = s;
   }
 }
 

@@ -229,17 +229,6 @@ struct MmArgs {
   int64_t y_stride;
 };
 
-// The columns [c0, c1) of one dot product in fp32 from the decoded weights.  An
-// output whose matrix-core sum is NaN -- an infinite or NaN activation or
-// weight, or block sums that overflowed with both signs -- is formed again this way.
-template <int TYPE>
-G4_DEV float mm_plain_dot(const uint8_t *W, int64_t E, const float *x, int c0, int c1, int dim1) {
-  float s = 0.f;
-#pragma clang loop unroll(disable)
-  for (int c = c0; c < c1; ++c) s = __builtin_fmaf(dot_elem<TYPE>(W, E + c, c, dim1), x[c], s);
-  return s;
-}
-
 // Every load (the direct ones, which the compiler's own waits do not count, among
 // them) and LDS operation of the wave is done; then all waves meet.
 G4_DEV void mm_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -505,17 +494,24 @@ __global__ __launch_bounds__(MM_THREADS) void k_mm(MmArgs a) {
         bad |= redo<TYPE>(sum);
       }
     }
-  if (bad) {
-    // the lane reads its own outputs back and forms these again
-    const int64_t E = a.base + (int64_t)row * a.row_stride;
+  if (__builtin_amdgcn_ballot_w64(bad) == 0) return;
+  // each lane reads its own outputs back, and the wave forms these again
 #pragma clang loop unroll(disable)
-    for (int q = 0; q < 32; ++q) {
-      const int v = q & 15, tok = (t_base + 2 * wm + (q >> 4)) * 32 + 8 * (v >> 2) + 4 * j + (v & 3);
-      if (tok >= a.M) continue;
-      volatile float *o = out + (int64_t)tok * a.y_stride + row;
-      if (redo<TYPE>(*o))
-        *o = mm_plain_dot<TYPE>(a.W, E, a.x + (int64_t)tok * a.x_stride, 64 * s0, min(64 * s1, a.dim1), a.dim1);
+  for (int q = 0; q < 32; ++q) {
+    const int v = q & 15, tok_j = (t_base + 2 * wm + (q >> 4)) * 32 + 8 * (v >> 2) + (v & 3);  // of lane half 0
+    const int tok = tok_j + 4 * j;
+    const bool mine = tok < a.M && row < a.rows;
+    volatile float *o = out + (int64_t)(mine ? tok : 0) * a.y_stride + (mine ? row : 0);
+    float s = mine ? *o : 0.f;
+    const bool again = mine && redo<TYPE>(s);
+    const uint64_t todo = __builtin_amdgcn_ballot_w64(again);
+    for (int half = 0; half < 2; ++half) {
+      const uint64_t lanes = todo & (0xFFFFFFFFull << (32 * half));
+      if (lanes)
+        form_again<TYPE>(a.W, a.base + (int64_t)(row - n) * a.row_stride, a.row_stride, 32 * half, lanes,
+                         a.x + (int64_t)(tok_j + 4 * half) * a.x_stride, 64 * s0, min(64 * s1, a.dim1), a.dim1, s);
     }
+    if (again) *o = s;
   }
 }
 

@@ -1128,15 +1128,16 @@ def _batched_case(g4, ctx, oracle, t, m, rows, dim1, off_rows):
     w.free()
 
 
+@pytest.mark.parametrize("dim1", [2048, 4224])
 @pytest.mark.parametrize("t", [Q8_0, Q4_0, Q5_K, Q6_K, BF16, F16])
-def test_batched_matrix_core_non_finite_and_wide_x(g4, ctx, oracle, t):
+def test_batched_matrix_core_non_finite_and_wide_x(g4, ctx, oracle, t, dim1):
     """Infinite and NaN activations reach their own tokens' outputs as in the sum of
     the products w * x (NaN for w = 0, else of the infinity's sign); a token spanning
     1e-20..1e20 and the finite tokens that share the waves stay within the bound."""
-    announce("batched non-finite x type %d" % t)
-    m, rows, dim1 = 12, 2056, 2048
-    raw = _no_subnormals(t, synth.weights(62, "mtn%d" % t, t, rows * dim1))
-    X = synth.activations(62, "mtnx", m * dim1).reshape(m, dim1)
+    announce("batched non-finite x type %d, %d columns" % (t, dim1))
+    m, rows = 12, 2056
+    raw = _no_subnormals(t, synth.weights(62, "mtn%d.%d" % (t, dim1), t, rows * dim1))
+    X = synth.activations(62, "mtnx%d" % dim1, m * dim1).reshape(m, dim1)
     X[4] *= (10.0 ** np.random.default_rng(62).uniform(-20, 20, dim1)).astype(np.float32)
     X[1, 5], X[2, 700], X[3, dim1 - 7] = np.inf, np.nan, -np.inf
     w = upload(g4, ctx, t, raw, rows * dim1)
