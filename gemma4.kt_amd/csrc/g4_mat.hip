@@ -206,7 +206,7 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
 
   float *out = gridDim.y == 1 ? a.y : a.part + (int64_t)blockIdx.y * a.M * a.rows;
   const int64_t out_stride = gridDim.y == 1 ? a.y_stride : a.rows;
-  uint64_t bad = 0;
+  RedoAny bad;
   for (int rt = rt0, buf = 0; rt < rt1; ++rt, buf ^= 1) {
     bf16x8 B[4];
     f32x4 sc[SPB == 2 ? 2 : 1];
@@ -304,10 +304,10 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
       const int r = rt * 16 + n, m = 4 * j + wid;
       const bool mine = r < a.rows && m < mt;
       if (mine) out[(int64_t)(tok0 + m) * out_stride + r] = s;
-      bad |= __builtin_amdgcn_ballot_w64(mine && redo<TYPE>(s));
+      bad.add(mine ? s : 0.f);
     }
   }
-  if (bad == 0) return;
+  if (__builtin_amdgcn_ballot_w64(bad.any()) == 0) return;
   // Waves 0..3: each lane reads its own outputs back, and the wave forms these again
   // (here and not where they are stored: in the loop it would cost registers, 19
   // tokens of Q8_0 14.2 -> 14.9 us, Q6_K 22.4 -> 25.3).
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
     const bool mine = r < a.rows && m < mt;
     volatile float *o = out + (int64_t)(tok0 + (mine ? m : 0)) * out_stride + (mine ? r : 0);
     float s = mine ? *o : 0.f;
-    const bool again = mine && redo<TYPE>(s);
+    const bool again = mine && redo(s);
     const uint64_t todo = __builtin_amdgcn_ballot_w64(again);
     for (int l0 = 0; l0 < 64; l0 += 16) {  // token 4 (l0 / 16) + wid
       const uint64_t lanes = todo & (0xFFFFull << l0);

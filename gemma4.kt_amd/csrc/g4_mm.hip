@@ -482,19 +482,17 @@ __global__ __launch_bounds__(MM_THREADS) void k_mm(MmArgs a) {
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int v = 0; v < 16; ++v) got[t][v] = in[(t * 16 + v) * 64];
-  bool bad = false;
+  RedoAny bad;
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const float sum = kh ? got[t][v] - acc[t][1][v] : acc[t][0][v] - got[t][v];
       const int tok = (t_base + 2 * wm + t) * 32 + 8 * (v >> 2) + 4 * j + (v & 3);
-      if (tok < a.M && row < a.rows) {
-        out[(int64_t)tok * a.y_stride + row] = sum;
-        bad |= redo<TYPE>(sum);
-      }
+      if (tok < a.M && row < a.rows) out[(int64_t)tok * a.y_stride + row] = sum;
+      bad.add(sum);  // (those past the end are zeros or a copy of the last row's)
     }
-  if (__builtin_amdgcn_ballot_w64(bad) == 0) return;
+  if (__builtin_amdgcn_ballot_w64(bad.any()) == 0) return;
   // each lane reads its own outputs back, and the wave forms these again
 #pragma clang loop unroll(disable)
   for (int q = 0; q < 32; ++q) {
@@ -503,7 +501,7 @@ __global__ __launch_bounds__(MM_THREADS) void k_mm(MmArgs a) {
     const bool mine = tok < a.M && row < a.rows;
     volatile float *o = out + (int64_t)(mine ? tok : 0) * a.y_stride + (mine ? row : 0);
     float s = mine ? *o : 0.f;
-    const bool again = mine && redo<TYPE>(s);
+    const bool again = mine && redo(s);
     const uint64_t todo = __builtin_amdgcn_ballot_w64(again);
     for (int half = 0; half < 2; ++half) {
       const uint64_t lanes = todo & (0xFFFFFFFFull << (32 * half));

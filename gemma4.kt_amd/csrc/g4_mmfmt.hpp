@@ -11,8 +11,9 @@
 //   BF16   the weight                   1                 --
 //   F16    the weight as two bf16 (8 and 3 significant bits)
 //
-// (The matrix cores do not take subnormal bf16 operands exactly: activations below
-// about 2^-110, whose smaller parts are subnormal, keep fewer significant bits.)
+// (The matrix cores do not take subnormal bf16 operands exactly: the smaller parts of
+// activations below about 2^-110 are.  Sums of nothing larger are formed again, see
+// redo(); activations that are themselves subnormal, below 2^-126, count as 0.)
 // Every integer has at most 8 significant bits, so the products with the three
 // bf16 parts of an fp32 activation are exact.  Scales are exact in fp32 (11 x 8
 // bits), and so are offsets.  Centred integers keep the sums' rounding at the
@@ -244,13 +245,28 @@ G4_DEV void f16_parts(const u32x4 &q, bf16x8 &hi, bf16x8 &lo) {
   lo = __builtin_bit_cast(bf16x8, b);
 }
 
-// A matrix-core sum that is formed again in fp32 from the decoded weights: NaN -- an
-// infinite or NaN activation or weight (an infinity's residual parts are NaN), or
-// block sums that overflowed with both signs -- and for F16 infinite (exponent 31).
-template <int TYPE>
+// A matrix-core sum that is formed again in fp32 from the decoded weights:
+//  - NaN or infinite: an infinite or NaN activation or weight (an infinity's residual
+//    parts are NaN; F16 exponent 31 is finite), or a block sum that overflowed, the
+//    integers being up to 128 times the weight's own scale;
+//  - below 2^-60, not 0: activations so small that their residual parts are subnormal,
+//    which the matrix cores do not take exactly.
 G4_DEV bool redo(float s) {
-  return TYPE == T_F16 ? !__builtin_isfinite(s) : s != s;
+  return !__builtin_isfinite(s) || (__builtin_fabsf(s) < 0x1p-60f && s != 0.f);
 }
+
+// Whether redo() holds for any of several sums, in four instructions each: the
+// largest and the smallest magnitude but 0 as integers (twice the bits, less one: 0
+// wraps to the largest).
+struct RedoAny {
+  uint32_t hi = 0u, lo = ~0u;
+  G4_DEV void add(float s) {
+    const uint32_t u = __float_as_uint(s) << 1;
+    hi = max(hi, u);
+    lo = min(lo, u - 1u);
+  }
+  G4_DEV bool any() const { return hi >= 0xFF000000u || lo < 0x42FFFFFFu; }
+};
 
 // The sums of one token (x, columns [c0, c1)) that the lanes of the set `lanes` hold
 // in s, lane l's that of row l - l0 of the rows from element E on: formed again one

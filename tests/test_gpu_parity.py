@@ -1152,6 +1152,31 @@ def test_batched_matrix_core_non_finite_and_wide_x(g4, ctx, oracle, t, dim1):
     w.free()
 
 
+@pytest.mark.parametrize("size", ["tiny", "huge"])
+@pytest.mark.parametrize("t,m,rows,dim1", [(t, 12, 2056, 2048) for t in (Q8_0, Q4_0, Q5_K, Q6_K, BF16, F16)] + [
+    (t, 512, 8192, 1024) for t in (Q8_0, Q4_0, Q4_K, Q6_K, F16)])
+def test_batched_matrix_core_extreme_x(g4, ctx, oracle, t, m, rows, dim1, size):
+    """Activations of about 1e-36, whose smaller bf16 parts are subnormal, and ones so
+    large that sum |w x| is 2e37 and a block's sum of integers times x overflows: the
+    sums stay within the bound, without its absolute part."""
+    announce("batched %s x type %d M=%d" % (size, t, m))
+    raw = _no_subnormals(t, synth.weights(62, "mte%d.%d" % (t, dim1), t, rows * dim1)).copy()
+    if size == "huge" and t not in (F16, BF16):  # small scales: integers far larger than the weights
+        block, at = {Q8_0: (34, (0,)), Q4_0: (18, (0,)), Q4_K: (144, (0, 2)), Q5_K: (176, (0, 2)), Q6_K: (210, (208,))}[t]
+        for k in at:
+            raw.reshape(-1, block)[:, k:k + 2] = np.array([1e-4], np.float16).view(np.uint8)
+    X = synth.activations(62, "mtex%d.%d" % (m, dim1), m * dim1).reshape(m, dim1)
+    _, ab = oracle.matmul_exact(t, raw, X[0], rows, dim1)
+    X = (X * (1e-36 if size == "tiny" else 2e37 / float(np.max(ab)))).astype(np.float32)
+    w = upload(g4, ctx, t, raw, rows * dim1)
+    Y = w.matmul_batch(X, rows, dim1)
+    for i in (0, 1, m // 2, m - 1):
+        ex, ab = oracle.matmul_exact(t, raw, X[i], rows, dim1)
+        # (tiny: a product below 2^-126 is rounded to a multiple of 2^-149)
+        assert np.all(np.abs(Y[i] - ex) <= TOL * ab + dim1 * 2.0 ** -149), float(np.max(np.abs(Y[i] - ex) / ab))
+    w.free()
+
+
 def test_batched_matrix_core_infinite_weight(g4, ctx, oracle):
     """An infinite BF16 weight gives its row infinite outputs (not the NaN that an
     infinity times an activation's zero residual part would)."""
