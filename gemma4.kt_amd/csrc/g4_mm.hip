@@ -236,7 +236,7 @@ G4_DEV void mm_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barr
 // 1 KB from src (wave-uniform) + 16 * lane to LDS at byte offset `to` (wave-uniform).
 G4_DEV void mm_direct_load(const unsigned char *src, uint32_t to, uint32_t lane16) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(lane16), "s"(src)
-               : "memory");
+               : "memory", "m0");
 }
 
 template <int TYPE>
