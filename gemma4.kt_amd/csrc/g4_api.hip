@@ -200,7 +200,9 @@ int zero_dev(g4_ctx *ctx, void *p, size_t bytes) {
 // or no memory is left.  A change of stream waits on the GPU: for an event recorded
 // behind the last use if that was on a caller's stream (which may be gone by now,
 // its handle another stream's), else for one recorded on own_stream here.
-char *ws_acquire(g4_ctx *ctx, size_t bytes) {
+// It grows to at least `least`.
+constexpr size_t WS_LEAST = size_t(64) << 20, WS_RESERVED = size_t(128) << 20;
+char *ws_acquire(g4_ctx *ctx, size_t bytes, size_t least = WS_LEAST) {
   if (ctx->capturing) return nullptr;
   // another thread's capture is not disturbed by the allocation and the waits
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -223,7 +225,7 @@ char *ws_acquire(g4_ctx *ctx, size_t bytes) {
       if (ctx->ws) (void)hipFree(ctx->ws);
       ctx->ws = nullptr;
       ctx->ws_bytes = 0;
-      const size_t want = std::max(bytes, size_t(64) << 20);
+      const size_t want = std::max(bytes, least);
       void *p = nullptr;
       ok = hipMalloc(&p, want) == hipSuccess;
       if (ok) {
@@ -963,7 +965,11 @@ int g4_ctx_reserve(g4_ctx *ctx, int64_t bytes) {
   G4_TRY(check_ctx(ctx));
   if (bytes < 0) return fail(G4_ERR_INVALID_ARGUMENT, "negative reservation %lld", (long long)bytes);
   G4_TRY(use_device(ctx));
-  return ensure_scratch(ctx, (size_t)bytes);
+  G4_TRY(ensure_scratch(ctx, (size_t)bytes));
+  // the several-token calls' workspace as well (they can do without it)
+  const size_t ws = std::min((size_t)bytes, WS_RESERVED);
+  if (ws > ctx->ws_bytes) (void)ws_acquire(ctx, ws, 0);
+  return G4_OK;
 }
 
 int g4_ctx_scratch_bytes(const g4_ctx *ctx, int64_t *bytes) {

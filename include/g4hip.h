@@ -89,7 +89,16 @@ int g4_ctx_device(const g4_ctx *ctx, int *ordinal);
  *    returns G4_ERR_INVALID_ARGUMENT and records nothing (g4_matmul_batch_dev of
  *    the types other than Q4_K then records its slower kernels, which need none);
  *  - once any call on the context has been captured, an outgrown buffer is kept
- *    allocated (graphs may still replay into it) until g4_close.
+ *    allocated (graphs may still replay into it) until g4_close;
+ *  - graphs of one context, and calls on it that use the buffer, run one after the
+ *    other, or on a context each.
+ * Eager g4_matmul_batch* calls (of more than 64 tokens, and for the types other
+ * than Q4_K of several tokens on rows of more than 2048 columns) use a second
+ * buffer, at least 64 MB from the first such call on, that no graph refers to and
+ * whose users on different streams are ordered by the library.  g4_ctx_reserve
+ * also readies as much of it, up to 128 MB; g4_ctx_scratch_bytes does not count
+ * it.  Where it cannot be had, and under capture, more than 64 tokens run on the
+ * 16-token kernels: fp32 sums in another order, and slower on long prompts.
  * Host-pointer calls synchronise and return G4_ERR_INVALID_ARGUMENT under capture.
  * No counterpart in the reference (its matmul is synchronous CPU code). */
 int g4_ctx_reserve(g4_ctx *ctx, int64_t bytes);

@@ -336,3 +336,26 @@ def test_shapes_meant_for_the_grouped_experts_take_them(hip):
     with Program(hip) as p:
         for E, D, FF, K, T, *_ in gpu.MOE_STRETCHES:
             assert p.moe(E, D, FF, K, T).count("k_grp_q4k") == 2, (E, D, FF)
+
+
+def test_a_reservation_covers_the_workspace(hip):
+    """A program that reserved up front meets no allocation and no wait of the host in
+    its first prompt."""
+    with Program(hip) as p:
+        for t, m, rows, cols in MANY + WIDE[:2]:
+            p.weight(t, rows * cols)
+        assert hip.g4_ctx_reserve(p.ctx, 256 << 20) == 0
+        hip.stub_clear()
+        s = p.stream()
+        for k, c in enumerate(MANY + WIDE[:2] + MANY):
+            p.use((None, s)[k % 2])
+            assert p.batch(*c)[0] in ("k_split", "k_mat")
+        assert not [l for l in p.log() if l[0] in ("malloc", "free", "sync", "sync_event", "sync_device")]
+        p.assert_ordered()
+
+
+def test_a_reservation_without_memory_for_the_workspace(hip):
+    with Program(hip) as p:
+        hip.stub_free_bytes(40 << 20)
+        assert hip.g4_ctx_reserve(p.ctx, 32 << 20) == 0
+        assert hip.stub_last_error() == 0
