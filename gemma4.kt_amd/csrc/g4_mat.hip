@@ -207,6 +207,7 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
   float *out = gridDim.y == 1 ? a.y : a.part + (int64_t)blockIdx.y * a.M * a.rows;
   const int64_t out_stride = gridDim.y == 1 ? a.y_stride : a.rows;
   RedoAny bad;
+  uint64_t bad_min = 0;  // (MIN has no registers left for it: 512 tokens of Q5_K 143 us, 124 so)
   for (int rt = rt0, buf = 0; rt < rt1; ++rt, buf ^= 1) {
     bf16x8 B[4];
     f32x4 sc[SPB == 2 ? 2 : 1];
@@ -304,10 +305,13 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(4, 4))
       const int r = rt * 16 + n, m = 4 * j + wid;
       const bool mine = r < a.rows && m < mt;
       if (mine) out[(int64_t)(tok0 + m) * out_stride + r] = s;
-      bad.add(mine ? s : 0.f);
+      if constexpr (MIN)
+        bad_min |= __builtin_amdgcn_ballot_w64(mine && redo(s));
+      else
+        bad.add(mine ? s : 0.f);
     }
   }
-  if (__builtin_amdgcn_ballot_w64(bad.any()) == 0) return;
+  if ((MIN ? bad_min : __builtin_amdgcn_ballot_w64(bad.any())) == 0) return;
   // Waves 0..3: each lane reads its own outputs back, and the wave forms these again
   // (here and not where they are stored: in the loop it would cost registers, 19
   // tokens of Q8_0 14.2 -> 14.9 us, Q6_K 22.4 -> 25.3).
