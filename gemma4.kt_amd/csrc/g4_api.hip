@@ -577,10 +577,11 @@ int check_moe(g4_ctx *ctx, const g4_weight *wgu, const g4_weight *wdn, int32_t T
 // Routing done inside the gate+up launch (g4_moe_routed*): the router logits in,
 // the ids and weights it stores out.
 // Calls of at least this many tokens run the experts grouped (launch_moe_grp):
-// measured on the 128-expert top-8 shape, the grouped launches take 174, 200, 213,
-// 220, 224, 226, 238 and 272 us at 16, 24, 32, 40, 48, 64, 128 and 200 tokens, the
-// per-pair ones 107, 151, 177 and 223 us at 16, 24, 32 and 40, 332 at 64 and 723 at
-// 128.
+// measured on the 128-expert top-8 shape (2048 x 1408), the grouped launches take
+// 155, 186, 203, 209, 216, 220, 227 and 266 us at 16, 24, 32, 40, 48, 64, 128 and 200
+// tokens, the per-pair ones 110, 155, 179, 223, 273, 324, 635 and 1158 us.  Fewer
+// experts or more slots cross earlier, more experts or fewer slots later: both
+// kernels' times go with the pairs per expert (four at 64 tokens here).
 constexpr int32_t MOE_GROUPED_MIN_T = 41;
 
 struct MoeRoute {

@@ -22,12 +22,12 @@
 // show (timing variants without them: 1-4% faster).  Measured at 8192 x 2048, us per
 // launch (one segment of the row engine per token -> here):
 //              8 tokens       19            64             512
-//   Q8_0     15.7 ->  9.9  45.9 -> 13.8   82.3 -> 21.7   625 -> 130
-//   Q4_0     13.3 ->  9.0                 72.4 -> 18.9
-//   Q5_K     18.9 -> 11.6  40.9 -> 15.5  109.1 -> 23.8
-//   Q6_K     24.6 -> 14.6  53.8 -> 20.1  141.8 -> 32.9
-//   BF16     32.5 -> 10.4  90.3 -> 11.8  227.6 -> 16.6  1786 -> 98.5
-//   F16      39.5 -> 16.4 100.7 -> 20.8  245.1 -> 32.0
+//   Q8_0     15.1 -> 10.0  46.5 -> 14.2   81.9 -> 23.6   623 -> 142
+//   Q4_0     12.0 ->  7.7  24.9 -> 10.8   71.6 -> 17.0   548 -> 113
+//   Q5_K     17.2 ->  9.8  39.7 -> 13.4  108.1 -> 21.3   833 -> 124
+//   Q6_K     23.1 -> 14.0  53.1 -> 20.4  140.5 -> 34.7   999 -> 216
+//   BF16     34.0 -> 10.8  90.5 -> 12.5  233.2 -> 19.2  1791 -> 98.9
+//   F16      40.2 -> 12.2 101.0 -> 15.6  247.9 -> 24.5  1898 -> 151
 // and against 64 bits the error falls from 1.2e-7..3.0e-7 to 0.7e-7..1.5e-7 (512 to
 // 32768 columns).
 #include "g4_mmfmt.hpp"

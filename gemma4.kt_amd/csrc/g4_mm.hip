@@ -575,13 +575,13 @@ hipError_t mm_launch(const MmArgs &a, hipStream_t s) {
 // is about 5 us before the first row tile and, per tile of 16 waves, the time
 // below (16 M weights, 512 tokens).  Measured, us, 16-token tiles / here:
 //                          100 tokens    201         320         512
-//   Q8_0  8192 x 2048     34.0 / 30.3  58 / 42.4   87 / 69.5  129 / 76.0
-//   Q4_0  8192 x 2048     28.1 / 31.6  48 / 41.3   69 / 68.1  100 / 74.0
-//   Q4_0  2048 x 8192     32.9 / 30.8  57 / 42.0   75 / 67.5  106 / 87.7
-//   Q4_K  8192 x 2048     22.6 / 32.3  37 / 42.9   52 / 59.4   75 / 65.1
-//   Q6_K  8192 x 2048     53.6 / 33.1  93 / 46.1  140 / 65.5  203 / 70.9
-//   F16   8192 x 2048     63.2 / 37.0 116 / 56.8  169 / 96.8  249 / 110 (f16_parts since faster: 54.2, 111 here)
-//   Q8_0  2048 x 2048     13.1 / 22.7  20 / 24.8   27 / 29.2   38 / 31.4
+//   Q8_0  8192 x 2048     37.9 / 30.0  65 / 42.5   95 / 72.4  142 / 79.9
+//   Q4_0  8192 x 2048     27.5 / 31.6  51 / 40.9   77 / 76.8  113 / 78.1
+//   Q4_0  2048 x 8192     32.8 / 32.4  62 / 42.4   83 / 68.6  119 / 89.0
+//   Q4_K  8192 x 2048     21.4 / 32.3  36 / 42.9   52 / 59.4   77 / 65.9
+//   Q6_K  8192 x 2048     56.6 / 31.9  99 / 45.4  147 / 66.1  216 / 71.3
+//   F16   8192 x 2048     39.9 / 36.2  70 / 54.3  103 / 94.2  151 / 107
+//   Q8_0  2048 x 2048     13.0 / 22.7  20 / 24.8   27 / 29.2   38 / 31.4
 // Q4_K over 408 shapes of 65 to 1024 tokens, 512 to 16384 rows and 512 to 8192
 // columns: never more than 3% slower than k_tok_q4k (4096 x 512, 256 tokens 17.6 /
 // 24.5; 5000 x 1024, 320 tokens 26.6 / 31.7; 16384 x 512, 512 tokens 106 / 42.8).
@@ -594,7 +594,8 @@ static bool mm_faster(int type, const TokArgs &a, const DevInfo &dev) {
     case T_Q4_0: tile = 1.5; break;
     // (of 1024 columns and fewer, half of the waves or more have none)
     case T_Q4_K: tile = a.dim1 <= 1024 ? 0.78 : 1.1; break;
-    default: tile = 3.1; break;  // Q6_K, F16
+    case T_F16: tile = 2.3; break;
+    default: tile = 3.1; break;  // Q6_K
   }
   const int n_sl = (a.dim1 + 127) / 128, splits = (n_sl + 15) / 16, sps = (n_sl + splits - 1) / splits;
   const int wpb = type == T_Q4_K ? 16 : sps <= 4 ? 4 : sps <= 8 ? 8 : 16, n_rt = (a.rows + 15) / 16;
@@ -672,8 +673,8 @@ hipError_t launch_mm(int type, const TokArgs &t, void *ws, const DevInfo &dev, h
         case T_Q8_0: e = mm_launch<T_Q8_0>(a, s); break;
         case T_Q4_0: e = mm_launch<T_Q4_0>(a, s); break;
         case T_Q4_K: e = mm_launch<T_Q4_K>(a, s); break;
-          case T_Q6_K: e = mm_launch<T_Q6_K>(a, s); break;
-          default: e = mm_launch<T_F16>(a, s); break;
+        case T_Q6_K: e = mm_launch<T_Q6_K>(a, s); break;
+        default: e = mm_launch<T_F16>(a, s); break;
       }
       if (e != hipSuccess) return e;
       if (p.splits > 1) {

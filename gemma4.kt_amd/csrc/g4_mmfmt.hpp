@@ -113,7 +113,6 @@ template <>
 struct MmFmt<T_Q8_0> {
   static constexpr int SPB = 1;  // scales per block
   static constexpr bool MIN = false;
-  static constexpr int UNIT = 32;
   u32x4 q[2];
   uint32_t d;
   G4_DEV static const uint8_t *at(const uint8_t *W, int64_t e) { return W + (e >> 5) * 34; }
@@ -135,7 +134,6 @@ template <>
 struct MmFmt<T_Q4_0> {
   static constexpr int SPB = 1;
   static constexpr bool MIN = false;
-  static constexpr int UNIT = 32;
   u32x4 q;
   uint32_t d;
   G4_DEV static const uint8_t *at(const uint8_t *W, int64_t e) { return W + (e >> 5) * 18; }
@@ -161,7 +159,6 @@ template <>
 struct MmFmt<T_Q5_K> {
   static constexpr int SPB = 1;
   static constexpr bool MIN = true;
-  static constexpr int UNIT = 128;
   u32x4 q, b, H;
   G4_DEV static const uint8_t *at(const uint8_t *W, int64_t e) { return W + (e >> 8) * 176; }
   G4_DEV void load(const uint8_t *p, int h, int, int i) {
@@ -198,7 +195,6 @@ template <>
 struct MmFmt<T_Q6_K> {
   static constexpr int SPB = 2;
   static constexpr bool MIN = false;
-  static constexpr int UNIT = 128;
   u32x4 q, b;
   uint32_t d, sc;
   G4_DEV static const uint8_t *at(const uint8_t *W, int64_t e) { return W + (e >> 8) * 210; }
@@ -226,7 +222,8 @@ struct MmFmt<T_Q6_K> {
 // other 3 (the difference is exact).  Subnormals are 0, as in the vector path
 // (h2f_vec).  Exponent 31, finite there, is infinite or NaN here and makes every
 // sum it enters so: the caller forms such sums again.  (8192 x 2048, 19 and 64
-// tokens: 24.2 and 38.5 us with h2f_vec's decode of each weight, 20.8 and 32.0 so.)
+// tokens: 24.2 and 38.5 us with h2f_vec's decode of each weight, 20.8 and 32.0 so,
+// before the parts were made two blocks at a time.)
 G4_DEV void f16_parts(const u32x4 &q, bf16x8 &hi, bf16x8 &lo) {
   u32x4 a, b;
 #pragma unroll

@@ -959,7 +959,10 @@ __global__ __launch_bounds__(MG_WPB * 64) void k_moe_grp(MoeGrpArgs a) {
 // more than 16 pairs ran their second pass: 200 tokens, 128 experts, top-8,
 // 431 -> 264 us a call; 41 tokens, 32 experts, top-8, ff 704, 128 -> 69 us.)
 constexpr int GT_WPB = 16;
-constexpr int GT_MAX_E = GT_WPB * 64;  // experts: one thread each
+// Experts: one thread each.  With more, a call has at most four pairs per expert
+// (MG_MAX_S), and k_moe_grp takes less: 1100 experts of 1024 x 256, top-8, 64 and 200
+// tokens 135 and 221 us there, 209 and 416 us with these tiles.
+constexpr int GT_MAX_E = GT_WPB * 64;
 
 template <bool AL>
 __global__ __launch_bounds__(GT_WPB * 64) void k_grp_q4k(MoeGrpArgs a) {
