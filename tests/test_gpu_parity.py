@@ -1236,13 +1236,17 @@ def test_moe_grouped_equal_stretches(g4, ctx, oracle, E, D, FF, K, T, skew, drop
 
 
 # Many tokens in tiles of 128 (k_mm; rows and columns large enough that it is the
-# faster route): rows that are not whole tiles of 128, one to three token tiles
-# with a partial last one, an odd number of 64-column stages and a last one of 32
-# columns (Q8_0, Q4_0), column splits, rows behind an offset.
-@pytest.mark.parametrize("t,m,rows,dim1,off_rows", [
-    (Q8_0, 130, 4100, 2112, 0), (Q8_0, 201, 2050, 4128, 1), (Q4_0, 300, 4000, 2080, 0), (Q4_K, 512, 8200, 2048, 0),
-    (Q4_K, 500, 2500, 4160, 1), (Q6_K, 129, 4099, 2048, 0), (Q6_K, 257, 2048, 2368, 2), (F16, 150, 4098, 2048, 0),
-    (F16, 257, 3000, 1088, 1)])
+# faster route, which tests/test_host_calls.py checks): rows that are not whole
+# tiles of 128, with column splits and without, one to four token tiles with a
+# partial last one, an odd number of 64-column stages and a last one of 32 columns
+# (Q8_0, Q4_0), rows behind an offset, and rows in three passes (more split sums
+# than are held at a time; the last pass has four rows).
+MM_SHAPES = [(Q8_0, 130, 4100, 2112, 0), (Q8_0, 201, 2050, 4128, 1), (Q4_0, 300, 4000, 2080, 0), (Q4_K, 512, 8100, 2048, 0),
+             (Q4_K, 500, 2500, 4160, 1), (Q6_K, 129, 4099, 2048, 0), (Q6_K, 257, 2048, 2368, 2), (F16, 200, 4098, 2048, 0),
+             (F16, 257, 3000, 1088, 1), (Q8_0, 1024, 4100, 8192, 0), (Q4_K, 510, 8189, 512, 0)]
+
+
+@pytest.mark.parametrize("t,m,rows,dim1,off_rows", MM_SHAPES + [(Q4_K, 512, 8200, 2048, 0)])
 def test_batched_many_tokens_shapes(g4, ctx, oracle, t, m, rows, dim1, off_rows):
     announce("batched many type %d M=%d rows=%d dim1=%d off_rows=%d" % (t, m, rows, dim1, off_rows))
     n, off = -(-(rows + off_rows) * dim1 // 256) * 256, off_rows * dim1
@@ -1261,7 +1265,7 @@ def test_batched_many_tokens_shapes(g4, ctx, oracle, t, m, rows, dim1, off_rows)
     w.free()
 
 
-@pytest.mark.parametrize("t", [Q8_0, Q4_K, Q6_K, F16])
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, Q4_K, Q6_K, F16])
 def test_batched_many_tokens_non_finite_and_wide_x(g4, ctx, oracle, t):
     """As for few tokens: infinities and NaN reach their own tokens' outputs as in
     the sum of the products; the others stay within the bound."""

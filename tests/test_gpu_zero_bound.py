@@ -209,3 +209,22 @@ def test_zero_rows_batched_many(g4, ctx, oracle, t):
         y64, ab = oracle.matmul_exact(t, raw, X[i], rows, cols)
         _check(Y[i], y64, ab, kinds, "batched token %d" % i)
     w.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", [Q4_0, Q4_K])
+def test_zero_rows_tiled_product(g4, ctx, oracle, t):
+    """512 tokens in tiles of 128: the integers are 0 where the weight is, and Q4_K's
+    offset 8 d sc - dmin m is formed exactly."""
+    announce("zero-bound tiled product type %d" % t)
+    rows, cols, m = 8192, 512, 512
+    kinds = _kinds(rows)
+    raw = BUILD[t](rows, cols, kinds)
+    X = synth.activations(9, "X%d" % m, m * cols).reshape(m, cols)
+    w = g4.FloatTensorFactory.create(ctx, t, raw, rows * cols)
+    Y = w.matmul_batch(X, rows, cols)
+    for i in (0, 31, 64, 127, 128, 300, 511):
+        y64, ab = oracle.matmul_exact(t, raw, X[i], rows, cols)
+        _check(Y[i], y64, ab, kinds, "token %d" % i)
+    assert np.all(Y[:, [k == "zero" for k in kinds]] == 0.0)
+    w.free()

@@ -359,3 +359,18 @@ def test_a_reservation_without_memory_for_the_workspace(hip):
         hip.stub_free_bytes(40 << 20)
         assert hip.g4_ctx_reserve(p.ctx, 32 << 20) == 0
         assert hip.stub_last_error() == 0
+
+
+def test_shapes_meant_for_the_tiled_product_take_it(hip):
+    """The sizes at which tests/test_gpu_parity.py and its neighbours test k_mm."""
+    with Program(hip) as p:
+        cases = [c[:4] for c in gpu.MM_SHAPES]
+        cases += [(t, 512, 8192, 1024) for t in (Q8_0, Q4_0, Q4_K, Q6_K, F16)]
+        cases += [(t, 512, 8192, 512) for t in (Q4_0, Q4_K)]
+        cases += [(Q6_K, m, 8192, 2048) for m in (100, 300, 120, 1300, 200, 700)]
+        cases += [(Q8_0, 512, 512, 32768), (Q4_0, 300, 2048, 8192), (Q6_K, 512, 8192, 2048)]
+        for c in cases:
+            assert "k_mm" in p.batch(*c), c
+        assert p.batch(Q8_0, 1024, 4100, 8192).count("k_mm") == 3  # rows in passes
+        assert p.batch(Q6_K, 1300, 8192, 2048).count("k_split") == 2  # tokens in passes
+        assert p.batch(Q4_K, 512, 8100, 2048) == ["k_split", "k_mm"]  # no split
