@@ -247,7 +247,11 @@ char *ws_acquire(g4_ctx *ctx, size_t bytes, size_t least = WS_LEAST) {
 // The workspace's use is queued on the context's stream.
 int ws_release(g4_ctx *ctx) {
   ctx->ws_use = ctx->stream == ctx->own_stream ? g4_ctx::WS_OWN : g4_ctx::WS_CALLER;
-  if (ctx->ws_use == g4_ctx::WS_CALLER) G4_HIP(hipEventRecord(ctx->ws_event, ctx->stream), "hipEventRecord");
+  if (ctx->ws_use == g4_ctx::WS_CALLER && hipEventRecord(ctx->ws_event, ctx->stream) != hipSuccess) {
+    (void)hipGetLastError();
+    G4_HIP(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");  // no event to order the next use by
+    ctx->ws_use = g4_ctx::WS_IDLE;
+  }
   return G4_OK;
 }
 
@@ -483,8 +487,9 @@ int batch_prepare(g4_ctx *ctx, const g4_weight *w, int64_t off, int32_t M, int32
     *r = {BatchRoute::ROWS, 0, nullptr};
   if (!ws) return ensure_scratch(ctx, before + sizeof(float) * (size_t)r->part);
   // Captured, the same call needs the scratch: an eager run of it leaves that (if
-  // there is the memory).
-  if (ensure_scratch(ctx, bytes) != G4_OK) (void)hipGetLastError();
+  // there is the memory).  Host-pointer calls, which have scratch besides, cannot be
+  // captured.
+  if (before == 0 && ensure_scratch(ctx, bytes) != G4_OK) (void)hipGetLastError();
   r->part = 0;
   r->ws = ws;
   return ensure_scratch(ctx, before);
